@@ -351,7 +351,7 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "pmc_k_rhs3_heat3d_p2_128.md")
 
 
 def launch_traffic(kernel):
-    """HBM bytes per launch of the element kernel `kernel` (k_rhs3, k_rhs3_pipe, k_rhs3_zpair) at 128^3
+    """HBM bytes per launch of the element kernel `kernel` (k_rhs3, k_rhs3_pipe, k_rhs3_march) at 128^3
     from the committed counter summary (the line `traffic_bytes_per_launch <kernel>: <bytes>`),
     or None when there is none."""
     key = f"traffic_bytes_per_launch {kernel}:"
@@ -519,11 +519,12 @@ def main():
     value = N * args.steps / t64
     ms_step = 1e3 * t64 / args.steps
 
-    # dominant kernel: the element kernel (k_rhs3; k_rhs3_pipe, k_rhs3_zpair for variants 3, 4),
+    # dominant kernel: the element kernel (k_rhs3; k_rhs3_pipe, k_rhs3_zpair for variants 3, 4,
+    # k_rhs3_march for variant 4 in one launch),
     # launched once over all tiles (tiling 1; its spill fix-up k_rhs_fixup runs at the start
     # of the sweep phase), or once per parity colour (8 launches per step, each over E/8
     # elements); HIP events on the handle's stream bracket the launches of the phase
-    rhs_kernel = {3: "k_rhs3_pipe", 4: "k_rhs3_zpair"}.get(var64, "k_rhs3")
+    rhs_kernel = {3: "k_rhs3_pipe", 4: "k_rhs3_march" if til64 == 1 else "k_rhs3_zpair"}.get(var64, "k_rhs3")
     one = til64 == 1 and var64 != 3
     launches = 1 if one else 8
     launch_flops = f_elem(3, 2) * E / launches
@@ -591,7 +592,7 @@ def main():
                                                 args.rhs_variant)
         ti, phi, xi, vari = run_increment_form(ag, ag.FP64, ne, args.steps, args.warmup, u0, dt)
         err = float(np.linalg.norm(x32 - x64) / np.linalg.norm(x64))
-        kern32 = {3: "k_rhs3_pipe", 4: "k_rhs3_zpair"}.get(var32, "k_rhs3")
+        kern32 = {3: "k_rhs3_pipe", 4: "k_rhs3_march" if til32 == 1 else "k_rhs3_zpair"}.get(var32, "k_rhs3")
         tf32 = f_elem(3, 2) * E / (ph32["rhs"] * 1e-3) / 1e12
         result["forms"] = {
             "fp64": {"value": value, "ms_per_step": ms_step},

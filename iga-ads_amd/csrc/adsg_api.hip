@@ -117,6 +117,13 @@ int upload_tables(adsg_sim* h, dev_dir& d) {
                 bval[k] = d.tab.val[k] * w;
                 bder[k] = d.tab.der[k] * w;
             }
+    std::vector<double> pack(h->dim == 3 ? static_cast<size_t>(d.tab.elements) * 4 * per : 0);
+    for (size_t i = 0; i < pack.size(); ++i) {
+        const size_t a = i % (d.tab.p + 1), r = i / (d.tab.p + 1), k = (r / 4) * (d.tab.p + 1) + a;
+        pack[i] = r % 4 == 0 ? val[k] : r % 4 == 1 ? der[k] : r % 4 == 2 ? bval[k] : bder[k];
+    }
+    if (h->dim == 3 && (rc = h->precision == ADSG_FP32 ? upload<float>(h, &d.pack, pack) : upload<double>(h, &d.pack, pack)))
+        return rc;
     if (h->precision == ADSG_FP32) {
         if ((rc = upload<float>(h, &d.val, val))) return rc;
         if ((rc = upload<float>(h, &d.der, der))) return rc;
@@ -150,6 +157,7 @@ void dir_tables(const adsg_sim* h, adsg::dev_tables<TT>* t) {
         t[d].wj = static_cast<const TT*>(h->dirs[d].wj);
         t[d].bval = static_cast<const TT*>(h->dirs[d].bval);
         t[d].bder = static_cast<const TT*>(h->dirs[d].bder);
+        t[d].pack = static_cast<const TT*>(h->dirs[d].pack);
         t[d].elements = h->dirs[d].tab.elements;
         t[d].dofs = h->dirs[d].tab.dofs;
         t[d].first = h->dirs[d].first;
@@ -168,7 +176,8 @@ hipError_t launch_elements(const adsg_sim* h, const T* up, T* out, const adsg::d
                            adsg::rhs_fixup<T>* defer = nullptr) {
     if (h->general) {
         if (overwrite) {
-            const hipError_t e = adsg::launch_fill<T>(out, h->N, T(0), h->stream);
+            const hipError_t e = prm.start ? adsg::launch_scale<T>(out, prm.start, h->N, prm.start_scale, h->stream)
+                                           : adsg::launch_fill<T>(out, h->N, T(0), h->stream);
             if (e != hipSuccess) return e;
         }
         return adsg::launch_rhs_general<T>(h->dim, up, out, t, prm, h->stream);
@@ -357,8 +366,8 @@ int sweep_all(adsg_sim* h, T* u, const int* slots, int mode = 0, const adsg::rhs
 
 // delta: the integrand exactly as given, from u_prev (its FP32 shadow in FP32 mode) into
 // buffer; otherwise compute_rhs semantics (FP64: into u; FP32: rhs - M u_prev into buffer)
-// b_i = sum_e sum_q w J f(x_q) B_i(x_q) for the source f: the element kernel with the
-// form {mass 0, dt 1, no gradient, source f}, in the step precision
+// b_i = sum_e sum_q w J f(x_q) B_i(x_q) for the source f, in the step precision: f is a spline
+// on the same basis, so this is the element loop's mass term applied to its coefficients
 template <typename T>
 int source_load_impl(adsg_sim* h) {
     if (!h->source_load && hipMalloc(&h->source_load, h->N * sizeof(T)) != hipSuccess)
@@ -366,14 +375,10 @@ int source_load_impl(adsg_sim* h) {
     adsg::dev_tables<T> t[3];
     dir_tables(h, t);
     adsg::rhs_params<T> prm;
-    prm.mass = T(0);
-    prm.dt = T(1);
-    prm.gx = prm.gy = prm.gz = T(0);
-    prm.source = static_cast<const T*>(h->vec[ADSG_SOURCE]);
+    prm.mass = T(1);
+    prm.dt = prm.gx = prm.gy = prm.gz = T(0);
     T* b = static_cast<T*>(h->source_load);
-    hipError_t e = adsg::launch_fill<T>(b, h->N, T(0), h->stream);
-    if (e == hipSuccess)
-        e = launch_elements<T>(h, prm.source, b, t, prm);
+    const hipError_t e = launch_elements<T>(h, static_cast<const T*>(h->vec[ADSG_SOURCE]), b, t, prm, true);
     if (e != hipSuccess) return hip_fail(h, e, "source load vector");
     h->source_load_ok = true;
     return ADSG_OK;
@@ -420,11 +425,15 @@ int rhs_impl(adsg_sim* h, const adsg_rhs_form* form, bool delta = false, adsg::r
     // entry, so only a source needs a start value
     const bool kron = h->rhs_kron && h->dim == 3 && !h->general && !form->use_kfield && form->reaction == 0.0;
     hipError_t e = hipSuccess;
-    // zero(rhs): done by the element launch (launch_elements with overwrite), which needs no
-    // fill in the one-launch tiling
-    if (form->use_source)
+    // the start value (zero, or dt times the source's load vector) is written by the element
+    // launch (launch_elements with overwrite), in one-launch tilings without a pass of its own
+    if (form->use_source && kron)
         e = adsg::launch_scale<T>(rhs, static_cast<const T*>(h->source_load), h->N, prm.dt, h->stream);
     if (e != hipSuccess) return hip_fail(h, e, "rhs start");
+    if (form->use_source) {
+        prm.start = static_cast<const T*>(h->source_load);
+        prm.start_scale = prm.dt;
+    }
     mark(h, 1);
     if (kron) {
         adsg::kron_dir kd[3];
@@ -438,7 +447,7 @@ int rhs_impl(adsg_sim* h, const adsg_rhs_form* form, bool delta = false, adsg::r
         e = adsg::launch_rhs_kron<T>(h->dim, h->dirs[0].tab.p, up, rhs, kd, mass, form->dt, form->grad,
                                      form->use_source, h->stream);
     } else {
-        e = launch_elements<T>(h, up, rhs, t, prm, !form->use_source, defer);
+        e = launch_elements<T>(h, up, rhs, t, prm, true, defer);
     }
     if (e != hipSuccess) return hip_fail(h, e, "rhs assembly");
     mark(h, 2);
@@ -632,9 +641,8 @@ int apply_linear_form(adsg_sim* h, const adsg_rhs_form* form, const double* v, d
         mark(h, 2);
         return ADSG_OK;
     }
-    if ((e = adsg::launch_fill<double>(out, h->N, 0.0, h->stream)) != hipSuccess) return hip_fail(h, e, "zero");
     mark(h, 1);
-    e = launch_elements<double>(h, v, out, t, prm);
+    e = launch_elements<double>(h, v, out, t, prm, true);
     if (e != hipSuccess) return hip_fail(h, e, "rhs assembly");
     mark(h, 2);
     return ADSG_OK;
@@ -659,9 +667,7 @@ int gram_apply(adsg_sim* h, const double* v, double* out) {
         adsg::rhs_params<double> prm;
         prm.mass = 1.0;
         prm.dt = 0.0;
-        e = adsg::launch_fill<double>(out, h->N, 0.0, h->stream);
-        if (e == hipSuccess)
-            e = launch_elements<double>(h, v, out, t, prm);
+        e = launch_elements<double>(h, v, out, t, prm, true);
     }
     return e == hipSuccess ? ADSG_OK : hip_fail(h, e, "Gram product");
 }
@@ -974,11 +980,15 @@ int adsg::create_sim(const adsg_config* cfg, hipStream_t shared, bool vectors, a
         h->dirs[d].slots.push_back(std::move(s0));
     }
     // default element-kernel variant (adsg_autotune refines it): the one measured fastest for
-    // the degree and precision. p = 3: FP64 2 (variants 0 and 1 need more registers than allow
-    // two waves per SIMD), FP32 5 (element columns on the matrix cores); p <= 2: 4 from 2^21
-    // elements (enough tiles of 512 elements to fill the device twice over), else 1. 3D
-    // handles start with the one-launch tiling (ADSG_TUNE_RHS_TILING), which was faster for
-    // every variant measured (p = 2 at 128^3, p = 3 at 192^3, both precisions); so do 2D
+    // the degree, precision and size. In one launch variant 4 is the marching kernel: a tile of
+    // it marches through its elements plane by plane, so it needs elements enough to fill the
+    // device with short marches; below, the per-element kernels finish sooner. Crossovers (step
+    // times, cubes and 77 x 101 x 61): p = 3 between 40^3 (FP64 variant 2 27 against 31 us per
+    // element pass, FP32 variant 1 20 against 23) and 48^3 (60 against 50, 37 against 29); p = 2
+    // FP64 between 64^3 (31 against 34) and 77 x 101 x 61 (60 against 57), FP32 between 96^3 (55
+    // against 58) and 128^3 (113 against 88); p = 1 between 96^3 (31 against 31; FP32 22 against
+    // 24) and 128^3 (59 against 53; 38.2 against 37.7). 3D handles start with the one-launch
+    // tiling (ADSG_TUNE_RHS_TILING), which was faster for every variant measured; so do 2D
     // handles of at most 2048 tiles of 16 x 16 elements, whose colour launches are too small to
     // fill the device (128^2 p = 2 with a k field: 0.046 -> 0.029 ms per step). Larger 2D
     // meshes keep the colour launches, as the batches do (with thousands of tiles per launch
@@ -987,7 +997,9 @@ int adsg::create_sim(const adsg_config* cfg, hipStream_t shared, bool vectors, a
         long E = 1;
         for (int d = 0; d < h->dim; ++d) E *= h->dirs[d].tab.elements;
         const int p = dc[0]->p;
-        h->rhs_variant = p == 3 ? (h->precision == ADSG_FP32 ? 5 : 2) : E >= (1L << 21) ? 4 : 1;
+        const bool f32 = h->precision == ADSG_FP32;
+        const long march = p == 3 ? 1L << 16 : f32 ? 1L << 20 : p == 2 ? 3L << 17 : 1L << 20;
+        h->rhs_variant = E >= march ? 4 : p == 3 && !f32 ? 2 : 1;
         h->rhs_col_shape = 1;  // variant 5: two columns per wave, one chunk per workgroup
         const long tiles16 = static_cast<long>((h->dirs[0].tab.elements + 15) / 16) * ((h->dirs[1].tab.elements + 15) / 16);
         h->rhs_tiling = h->general ? 0 : h->dim == 3 || tiles16 <= 2048 ? 1 : 0;
@@ -1115,7 +1127,7 @@ void adsg_destroy(adsg_sim* h) {
     drop_graphs(h);
     for (auto& d : h->dirs) {
         for (auto& s : d.slots) free_slot(s, h->in_arena);
-        for (void** p : {&d.val, &d.der, &d.wj, &d.bval, &d.bder, &d.rows, &d.kM, &d.kK})
+        for (void** p : {&d.val, &d.der, &d.wj, &d.bval, &d.bder, &d.pack, &d.rows, &d.kM, &d.kK})
             if (*p && !h->in_arena) (void)hipFree(*p);
         if (d.first && !h->in_arena) (void)hipFree(d.first);
     }

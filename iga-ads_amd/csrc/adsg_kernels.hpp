@@ -118,6 +118,8 @@ struct dev_tables {
     const T* wj = nullptr;
     const T* bval = nullptr;
     const T* bder = nullptr;
+    // the four tables of an element together, [elements][Gauss point][val, der, bval, bder][p+1]
+    const T* pack = nullptr;
     int elements = 0;
     int dofs = 0;
     const int* first = nullptr;  // first DOF of every element (general element loop)
@@ -147,6 +149,10 @@ struct rhs_params {
     // the one-launch tiling, and the first colour to reach a DOF in the 2D colour launches,
     // store their entries instead of adding them
     bool store = false;
+    // the start value of the rhs is start_scale * start (the load vector of a source) instead
+    // of what rhs holds: rhs := start_scale * start + the element sums
+    const T* start = nullptr;
+    T start_scale = 1;
 };
 
 // variant: kernel tuning choice (0 = coefficient block held in registers, 1 = re-read from
@@ -183,6 +189,25 @@ bool rhs3_col_supported(int p, const rhs_params<T>& prm);
 template <typename T>
 hipError_t launch_rhs3_col(int p, const T* u_prev, T* rhs, const dev_tables<T>* dirs, const rhs_params<T>& prm,
                            int shape, hipStream_t s);
+
+// Variant 4 in one launch (adsg_rhs_march.hip): its tiles (elements per tile and tile counts
+// per direction) for degree p, values of `bytes` bytes, with or without a k field; and its
+// launch on them (prm: the spill layout of these tiles set; no source in the kernel).
+// Forms with a k field: not FP32 at p = 3, where the sums along z in FP32 were 10 to 22 % further
+// from FP64 than the per-element kernels' sums across elements in FP64 (10 heat steps, 64^3 and
+// 128 x 100 x 90); everywhere else its FP32 error is no larger than theirs.
+template <typename T>
+constexpr bool rhs3_march_kfield(int p) {
+    return sizeof(T) == sizeof(double) || p < 3;
+}
+// its 32-bit byte offsets within a plane of DOFs
+constexpr bool rhs3_march_fits(int bytes, long nx, long ny) {
+    return nx * ny * bytes < (1L << 32);
+}
+void rhs3_march_tiles(int p, int bytes, bool kfield, const int elements[3], int tile[3], int nt[3]);
+template <typename T>
+hipError_t launch_rhs3_march(int p, const T* u_prev, T* rhs, const dev_tables<T>* dirs, const rhs_params<T>& prm,
+                             const int tile[3], const int nt[3], hipStream_t s);
 
 // Batched 2D element kernels: one item per problem (degree p, no k field, no source).
 template <typename T>

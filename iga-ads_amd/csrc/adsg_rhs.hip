@@ -10,6 +10,7 @@
 
 #include <algorithm>
 
+#include "adsg_device.hpp"
 #include "adsg_kernels.hpp"
 
 namespace adsg {
@@ -34,24 +35,6 @@ namespace {
 // planes with LDS atomic adds: a wave's adds are executed in instruction order, so the sums
 // are deterministic, and waves never share a plane. One barrier later the planes of the
 // (P+1) waves that touch a DOF plane are added and the tile's block is added into the rhs.
-constexpr int kXcds = 8;  // MI355X: 8 accelerator complex dies, 32 CUs each
-
-// block b (dispatched to XCD b % 8) -> tile index, a bijection of [0, n) that gives every
-// XCD a contiguous range of tiles
-__device__ __forceinline__ int xcd_contiguous(int b, int n) {
-    const int per = n / kXcds, rem = n % kXcds;
-    const int x = b % kXcds, i = b / kXcds;
-    return x < rem ? x * (per + 1) + i : rem * (per + 1) + (x - rem) * per + i;
-}
-
-// A read of read-only, wave-uniform data through the constant address space: always a
-// scalar load, also after instructions the compiler must treat as memory writes.
-template <typename T>
-__device__ __forceinline__ T uniform_load(const T* p) {
-    using CT = const __attribute__((address_space(4))) T*;
-    return *(CT)(p);
-}
-
 template <typename T, int P, int VAR>
 constexpr int rhs3_waves() {  // minimum waves per SIMD the register allocation must allow
     return VAR == 0 ? 1 : VAR == 1 || VAR == 3 || VAR == 4 ? 2 : P == 3 ? 2 : sizeof(T) == sizeof(float) ? 4 : 3;
@@ -107,20 +90,6 @@ __device__ __forceinline__ block_sink<T> rhs3_sink(T* rhs, tile3 o, int ex, int 
         return {rhs, {o.ex0 / TX, o.ey0 / TY, o.ez0 / TZ}, {o.ex0 + TX >= ex, o.ey0 + TY >= ey, o.ez0 + TZ >= ez}};
     else
         return {rhs, {0, 0, 0}, {false, false, false}};
-}
-// index of a spilled entry in the spill arrays: array delta = dx + 2 dy + 4 dz, position
-// (cx, cy, cz) in its extents
-template <typename T>
-__device__ __forceinline__ long spill_index(const rhs_params<T>& prm, int dx, int dy, int dz, int cx, int cy,
-                                            int cz) {
-    const int delta = dx + 2 * dy + 4 * dz;
-    long off = 0;
-#pragma unroll
-    for (int j = 1; j < 8; ++j)
-        if (delta == j) off = prm.spill_off[j];  // selects: no dynamic index into the argument
-    const long ex = dx ? prm.spill_ext[0][1] : prm.spill_ext[0][0];
-    const long ey = dy ? prm.spill_ext[1][1] : prm.spill_ext[1][0];
-    return off + cx + ex * (cy + ey * cz);
 }
 // entry (bx, by, bz) of the block, DOF (gx, gy, gz) = g of the mesh
 template <bool ONE, int P, int TX, int TY, int TZ, typename T>
@@ -786,7 +755,7 @@ __global__ __launch_bounds__(TX* TY* TZ, 2) void k_rhs3_pipe(
 // taller tile re-reads fewer halo planes. Wave w owns the LDS planes of DOF planes 2w ..
 // 2w+P+1; the block add, the colouring and the one-launch tiling are those of the other
 // variants.
-template <typename T, int P, int TX, int TY, int TZ, bool KF, bool SRC, int FM, bool ONE>
+template <typename T, int P, int TX, int TY, int TZ, bool KF, bool SRC, int FM>
 __global__ __launch_bounds__(TX* TY*(TZ / 2), 2) void k_rhs3_zpair(
     const T* __restrict__ up, T* __restrict__ rhs, dev_tables<T> X, dev_tables<T> Y,
     dev_tables<T> Z, rhs_params<T> prm, int colour, int ntx2, int nty2) {
@@ -803,7 +772,7 @@ __global__ __launch_bounds__(TX* TY*(TZ / 2), 2) void k_rhs3_zpair(
     const int lx = tid % TX, ly = (tid / TX) % TY;
     const int w = __builtin_amdgcn_readfirstlane(tid / 64);
     const int t = xcd_contiguous(blockIdx.x, gridDim.x);
-    const tile3 o = rhs3_tile_of<ONE, TX, TY, TZ>(t, colour, ntx2, nty2);
+    const tile3 o = rhs3_tile<TX, TY, TZ>(t, colour, ntx2, nty2);
     rhs3_stage<NT>(S.b, o, up, X, Y, Z.dofs, prm, tid);
     for (int i = tid; i < NW * WP * PL; i += NT) S.acc[i] = 0.0;
     __syncthreads();
@@ -835,7 +804,7 @@ __global__ __launch_bounds__(TX* TY*(TZ / 2), 2) void k_rhs3_zpair(
                                        __HIP_MEMORY_SCOPE_WAVEFRONT);
     __syncthreads();
     // DOF plane k of the block collects plane k - 2w of the waves w with 0 <= k - 2w <= P+1
-    const block_sink<T> sink = rhs3_sink<ONE, TX, TY, TZ>(rhs, o, X.elements, Y.elements, Z.elements);
+    const block_sink<T> sink = rhs3_sink<false, TX, TY, TZ>(rhs, o, 0, 0, 0);
     for (int i = tid; i < NB; i += NT) {
         const int bxy = i % PL, bz = i / PL;
         const int gx = o.ex0 + bxy % BX, gy = o.ey0 + bxy / BX, gz = o.ez0 + bz;
@@ -846,7 +815,7 @@ __global__ __launch_bounds__(TX* TY*(TZ / 2), 2) void k_rhs3_zpair(
             if (pl >= 0 && pl < WP) sum += S.acc[(ww * WP + pl) * PL + bxy];
         }
         if (gx < X.dofs && gy < Y.dofs && gz < Z.dofs)
-            rhs3_put<ONE, P, TX, TY, TZ>(sink, prm, bxy % BX, bxy / BX, bz, gx, gy, gz,
+            rhs3_put<false, P, TX, TY, TZ>(sink, prm, bxy % BX, bxy / BX, bz, gx, gy, gz,
                                          gx + static_cast<long>(X.dofs) * (gy + static_cast<long>(Y.dofs) * gz), sum);
     }
 }
@@ -1261,12 +1230,6 @@ struct tile<3, 3> {
     static constexpr int X = 8, Y = 8, Z = 3;
 };
 
-// element layers per tile of a variant: variant 4 (p <= 2) uses tiles twice as tall
-template <int P, int VAR>
-constexpr int rhs3_tile_z() {
-    return VAR == 4 && P <= 2 ? 2 * tile<3, P>::Z : tile<3, P>::Z;
-}
-
 template <typename T, int P, bool KF, bool SRC, int FM, int VAR>
 hipError_t rhs3_colours(const T* up, T* rhs, const dev_tables<T>* d, const rhs_params<T>& prm,
                         hipStream_t s) {
@@ -1286,7 +1249,7 @@ hipError_t rhs3_colours(const T* up, T* rhs, const dev_tables<T>* d, const rhs_p
             const int ntz2 = (d[2].elements + TZ2 - 1) / TZ2, nz22 = (ntz2 - cz + 1) / 2;
             const long tiles2 = static_cast<long>(nx2) * ny2 * nz22;
             if (tiles2 > 0)
-                hipLaunchKernelGGL((k_rhs3_zpair<T, P, TL::X, TL::Y, TZ2, KF, SRC, FM, false>), dim3(tiles2),
+                hipLaunchKernelGGL((k_rhs3_zpair<T, P, TL::X, TL::Y, TZ2, KF, SRC, FM>), dim3(tiles2),
                                    dim3(NT), 0, s, up, rhs, d[0], d[1], d[2], prm, c, nx2, ny2);
         } else if constexpr (VAR == 3) {
             hipLaunchKernelGGL((k_rhs3_pipe<T, P, TL::X, TL::Y, TL::Z, KF, SRC, FM>),
@@ -1425,16 +1388,14 @@ long spill_layout(const int n[3], const int nt[3], long off[8], int ext[3][2]) {
     return total;
 }
 
-// One launch over all tiles (variants 0, 1, 2 and 4; 4 at p = 3 runs as 2), then the spill
-// fix-up over the DOFs.
+// One launch over all tiles (variants 0, 1 and 2), then the spill fix-up over the DOFs.
 template <typename T, int P, bool KF, bool SRC, int FM, int VAR>
 hipError_t rhs3_one(const T* up, T* rhs, const dev_tables<T>* d, const rhs_params<T>& prm, hipStream_t s) {
     using TL = tile<3, P>;
-    constexpr int V = VAR == 4 && P == 3 ? 2 : VAR, TZ = rhs3_tile_z<P, V>();
-    static_assert(V != 3 && V != 5, "variants 3 and 5 have no one-launch form");
+    static_assert(VAR <= 2, "the other variants have no one-launch form here");
     const int ntx = (d[0].elements + TL::X - 1) / TL::X;
     const int nty = (d[1].elements + TL::Y - 1) / TL::Y;
-    const int ntz = (d[2].elements + TZ - 1) / TZ;
+    const int ntz = (d[2].elements + TL::Z - 1) / TL::Z;
     const long tiles = static_cast<long>(ntx) * nty * ntz;
     if (tiles == 0) return hipSuccess;
     if (!prm.spill) return hipErrorInvalidValue;
@@ -1444,25 +1405,54 @@ hipError_t rhs3_one(const T* up, T* rhs, const dev_tables<T>* d, const rhs_param
     for (int i = 0; i < 3; ++i)
         if (n[i] != d[i].elements + P) return hipErrorInvalidValue;
     spill_layout<P>(n, nt, q.spill_off, q.spill_ext);
-    if constexpr (V == 4)
-        hipLaunchKernelGGL((k_rhs3_zpair<T, P, TL::X, TL::Y, TZ, KF, SRC, FM, true>), dim3(tiles),
-                           dim3(TL::X * TL::Y * TZ / 2), 0, s, up, rhs, d[0], d[1], d[2], q, 0, ntx, nty);
-    else
-        hipLaunchKernelGGL((k_rhs3<T, P, TL::X, TL::Y, TZ, KF, SRC, FM, V, true>), dim3(tiles),
-                           dim3(TL::X * TL::Y * TZ), 0, s, up, rhs, d[0], d[1], d[2], q, 0, ntx, nty);
+    hipLaunchKernelGGL((k_rhs3<T, P, TL::X, TL::Y, TL::Z, KF, SRC, FM, VAR, true>), dim3(tiles),
+                       dim3(TL::X * TL::Y * TL::Z), 0, s, up, rhs, d[0], d[1], d[2], q, 0, ntx, nty);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const int tl[3] = {TL::X, TL::Y, TZ};
+    const int tl[3] = {TL::X, TL::Y, TL::Z};
     return finish_one(prm, q, rhs, P, tl, nt, n, s);
 }
 
-// spill values of one launch of a variant (dofs = elements + P)
-template <int P, int VAR>
+// Variant 4 in one launch: the marching kernel (adsg_rhs_march.hip) on its own tiles, then
+// the spill fix-up over the DOFs.
+template <typename T, int P>
+hipError_t rhs3_march(const T* up, T* rhs, const dev_tables<T>* d, const rhs_params<T>& prm, hipStream_t s) {
+    const int el[3] = {d[0].elements, d[1].elements, d[2].elements};
+    int tl[3], nt[3];
+    if (el[0] <= 0 || el[1] <= 0 || el[2] <= 0) return hipSuccess;
+    if (!prm.spill) return hipErrorInvalidValue;
+    rhs3_march_tiles(P, sizeof(T), prm.kfield != nullptr, el, tl, nt);
+    rhs_params<T> q = prm;
+    const int n[3] = {d[0].dofs, d[1].dofs, d[2].dofs};
+    for (int i = 0; i < 3; ++i)
+        if (n[i] != d[i].elements + P) return hipErrorInvalidValue;
+    spill_layout<P>(n, nt, q.spill_off, q.spill_ext);
+    const hipError_t e = launch_rhs3_march<T>(P, up, rhs, d, q, tl, nt, s);
+    if (e != hipSuccess) return e;
+    return finish_one(prm, q, rhs, P, tl, nt, n, s);
+}
+
+// the largest spill total of the marching kernel's tiles over its precisions and forms
+template <int P>
+long rhs3_march_slots(const int elements[3]) {
+    const int n[3] = {elements[0] + P, elements[1] + P, elements[2] + P};
+    long most = 0;
+    for (int k = 0; k < 4; ++k) {
+        int tl[3], nt[3], ext[3][2];
+        long off[8];
+        rhs3_march_tiles(P, k & 1 ? 8 : 4, (k & 2) != 0, elements, tl, nt);
+        most = std::max(most, spill_layout<P>(n, nt, off, ext));
+    }
+    return most;
+}
+
+// spill values of one launch of variants 0 to 2 (dofs = elements + P)
+template <int P>
 long rhs3_one_slots(const int elements[3]) {
     using TL = tile<3, P>;
-    constexpr int TZ = rhs3_tile_z<P, VAR>();
     const int n[3] = {elements[0] + P, elements[1] + P, elements[2] + P};
-    const int nt[3] = {(elements[0] + TL::X - 1) / TL::X, (elements[1] + TL::Y - 1) / TL::Y, (elements[2] + TZ - 1) / TZ};
+    const int nt[3] = {(elements[0] + TL::X - 1) / TL::X, (elements[1] + TL::Y - 1) / TL::Y,
+                       (elements[2] + TL::Z - 1) / TL::Z};
     long off[8];
     int ext[3][2];
     return spill_layout<P>(n, nt, off, ext);
@@ -1610,7 +1600,7 @@ template <typename T, int P, int VAR>
 hipError_t rhs3_fields(const T* up, T* rhs, const dev_tables<T>* d, const rhs_params<T>& prm,
                        bool one, hipStream_t s) {
     // one launch (forms without a k field or a source in the kernel; checked by the caller)
-    if constexpr (VAR != 3) {
+    if constexpr (VAR <= 2) {
         if (one) {
             if (prm.reaction != T(0)) return rhs3_one<T, P, false, false, 1, VAR>(up, rhs, d, prm, s);
             if (prm.mass == T(0)) return rhs3_one<T, P, false, false, 2, VAR>(up, rhs, d, prm, s);
@@ -1630,21 +1620,35 @@ hipError_t rhs_fields(int dim, const T* up, T* rhs, const dev_tables<T>* d,
     const bool kf = prm.kfield != nullptr, src = prm.source != nullptr;
     // bits 4..7: the shape of variant 5; bit 8: one launch; bit 9: overwrite
     int variant = code & 15;
-    const bool overwrite = (code & kRhsOverwrite) != 0;
     if (dim == 3 && variant == 5 && !rhs3_col_supported<T>(P, prm)) variant = P == 3 ? 2 : 1;
     // element columns on the matrix cores where the form allows, else the degree's default
     // per-element variant
+    const bool march = dim == 3 && !src && rhs3_march_fits(sizeof(T), d[0].dofs, d[1].dofs) &&
+                       (!kf || rhs3_march_kfield<T>(P));
     const bool one = (code & kRhsOneLaunch) != 0 && prm.spill &&
-                     (dim == 2 || (variant != 3 && variant != 5 && !kf && !src));
+                     (dim == 2 || (variant != 3 && variant != 5 && !src && (!kf || march)));
+    // 3D in one launch: the marching kernel for variant 4 and for every form with a k field,
+    // which the per-element kernels take in colour launches only (70 x 50 x 61, p = 2, FP64: 34 us
+    // against 154 us in eight launches and a fill)
+    const bool marched = march && one && (kf || variant == 4);
+    if (one && dim == 3 && variant == 4 && !marched) variant = P == 3 ? 2 : 1;
+    const long n = static_cast<long>(d[0].dofs) * d[1].dofs * (dim == 3 ? d[2].dofs : 1);
+    bool overwrite = (code & kRhsOverwrite) != 0;
+    if (prm.start && !marched) {  // the marching kernel adds it as it writes its block
+        const hipError_t e = launch_scale<T>(rhs, prm.start, n, prm.start_scale, s);
+        if (e != hipSuccess) return e;
+        prm.start = nullptr;
+        overwrite = false;
+    }
     // overwrite: the one launch's owners store, and so do the first colour to reach a DOF in
     // the 2D colour launches; the 3D colour launches add into a zero fill
-    prm.store = overwrite && (one || dim == 2);
+    prm.store = overwrite && !prm.start && (one || dim == 2);
     if (overwrite && !one && dim != 2) {
-        const long n = static_cast<long>(d[0].dofs) * d[1].dofs * (dim == 3 ? d[2].dofs : 1);
         const hipError_t e = launch_fill<T>(rhs, n, T(0), s);
         if (e != hipSuccess) return e;
     }
     if (dim == 3) {
+        if (marched) return rhs3_march<T, P>(up, rhs, d, prm, s);
         if (variant == 5) return launch_rhs3_col<T>(P, up, rhs, d, prm, (code >> 4) & 15, s);
         if (variant == 1) return rhs3_fields<T, P, 1>(up, rhs, d, prm, one, s);
         if (variant == 2) return rhs3_fields<T, P, 2>(up, rhs, d, prm, one, s);
@@ -1776,11 +1780,11 @@ long rhs_spill_slots(int dim, int p, const int elements[3]) {
     }
     switch (p) {
         case 1:
-            return std::max({rhs3_one_slots<1, 1>(elements), rhs3_one_slots<1, 4>(elements)});
+            return std::max(rhs3_one_slots<1>(elements), rhs3_march_slots<1>(elements));
         case 2:
-            return std::max({rhs3_one_slots<2, 1>(elements), rhs3_one_slots<2, 4>(elements)});
+            return std::max(rhs3_one_slots<2>(elements), rhs3_march_slots<2>(elements));
         case 3:
-            return rhs3_one_slots<3, 1>(elements);
+            return std::max(rhs3_one_slots<3>(elements), rhs3_march_slots<3>(elements));
         default:
             return 0;
     }

@@ -308,12 +308,14 @@ int adsg_time_phases(adsg_sim* h, int nsteps, const adsg_rhs_form* form, const i
  * ADSG_TUNE_RHS_VARIANT selects the 3D element-kernel variant (0: element coefficients held
  * in registers, 1: re-read from LDS, 2: as 1 with the element's contribution added to LDS
  * per x Gauss point, 3: two tiles per workgroup, the second tile's data copied to LDS while
- * the first is integrated, integrated like 1 (like 2 at p = 3), 4: each wave integrates two
- * element layers and carries their shared DOF planes in registers (p <= 2; 2 at p = 3));
+ * the first is integrated, integrated like 1 (like 2 at p = 3), 4: the shared DOF planes of a
+ * wave's element layers carried in registers: in one launch a march over all layers of a tile
+ * whose x and y contractions are shared by the elements too, in colour launches two layers per
+ * wave (p <= 2; 2 at p = 3));
  * they compute the same sums (variants 2 and 4 add them in other orders; in FP64 variant 3
  * equals 1, or 2 at p = 3, bit for bit). A new handle starts with the variant measured
- * fastest for its degree and precision (p = 3: 2; FP64 p <= 2: 4 from 2^21 elements, else
- * 1; FP32: 1).
+ * fastest for its degree, precision and element count (4 from 2^16 elements at p = 3, 3 * 2^17
+ * at p = 2 in FP64 and 2^20 otherwise; below, 2 for FP64 p = 3 and else 1).
  * ADSG_TUNE_SWEEP_VARIANT selects the line sweep (0: lines cut into segments solved by
  * separate waves and joined through FP64-computed influence coefficients, where the factors
  * are unpivoted and the lines are 2..16 segments of at most 32 rows long (up to 512 DOFs),
@@ -335,8 +337,8 @@ int adsg_time_phases(adsg_sim* h, int nsteps, const adsg_rhs_form* form, const i
  * of elements along z, the x-y contractions on the matrix cores): bit 0 two columns per
  * wave, bit 1 three chunks of 16 DOF planes per workgroup; the autotuner times all four. */
 #define ADSG_TUNE_RHS_COLUMNS 4
-/* ADSG_TUNE_RHS_TILING (2D every form; 3D variants 0, 1, 2 and 4 with forms without a k
- * field or source in the kernel): 0 = 2^dim parity-colour launches, whose tiles share no
+/* ADSG_TUNE_RHS_TILING (2D every form; 3D variants 0, 1, 2 and 4; forms with a k field run
+ * variant 4's kernel then, in FP32 for p <= 2): 0 = 2^dim parity-colour launches, whose tiles share no
  * DOF; 1 = one launch over all tiles, each tile adding the entries of its DOF block that it
  * owns and storing the others in a spill array (allocated with the handle, about one to
  * three values per element), which a second kernel adds in a fixed order. Both are
