@@ -1,4 +1,5 @@
-// Device helpers shared by the element-loop kernels (adsg_rhs.hip, adsg_rhs_march.hip).
+// Device helpers shared by the element-loop kernels (adsg_rhs.hip, adsg_rhs_march.hip) and the segmented
+// line sweeps (adsg_seg.inc).
 #pragma once
 
 #include <hip/hip_runtime.h>
