@@ -246,7 +246,7 @@ def ensemble_block(ag, np, count, steps, dt):
                                            "bands, FP64 band LU and packed sweep rows "
                                            "(adsg_batch_prepare), computed on the device; the "
                                            "host lays out the arenas and uploads their descriptors")},
-                     "tile_shape": ["16x16", "8x8"][tile], "line_sweeps": lines,
+                     "tile_shape": ["strips", "8x8"][tile], "line_sweeps": lines,
                      "autotune_ms_per_step": list(map(float, tile_ms)),
                      "element_tflops": flops * steps / t / 1e12}
     err = max(float(np.linalg.norm(a - c) / np.linalg.norm(c)) for a, c in zip(out["fp32"], out["fp64"]))

@@ -552,7 +552,7 @@ class Batch:
         self._check(lib().adsg_batch_synchronize(self.h), "batch_synchronize")
 
     def set_tuning(self, value, key=TUNE_BATCH_TILE):
-        """TUNE_BATCH_TILE: element tile (0 = 16x16, 1 = 8x8); TUNE_SWEEP_VARIANT: 0 =
+        """TUNE_BATCH_TILE: element kernel (0 = strips, 1 = 8x8 tiles); TUNE_SWEEP_VARIANT: 0 =
         segmented line sweeps, 1 = one lane per line."""
         self._check(lib().adsg_batch_set_tuning(self.h, key, value), "batch_set_tuning")
 

@@ -2,11 +2,9 @@
 //
 // Every problem keeps its own 1D tables and FP64-computed factors (an adsg_sim without state
 // vectors), while the state of all problems lives in shared arenas, problem after problem.
-// One step is a fixed sequence of grouped launches over all problems: zero fill of the
-// arena, per degree p and parity colour one element-kernel launch whose blocks cover the
-// tiles of every problem of that degree, per degree one x-sweep and one y-sweep launch over
-// all their lines, and one elementwise update of the whole arena. The step sequences are
-// replayed from captured HIP graphs of at most 50 steps. The problems' set-up runs on the
+// One step is a fixed sequence of grouped launches over all problems: one element-kernel
+// launch whose blocks are the strips of every problem, one x-sweep and one y-sweep launch over
+// all their lines, the FP32 update as the y sweeps store. The step sequences are replayed from captured HIP graphs of at most 50 steps. The problems' set-up runs on the
 // device (adsg_batch_setup.hip): create tabulates every direction's basis in one launch,
 // prepare assembles the Gram bands, factors them and packs the sweep rows in two more; the
 // host only lays out the arenas and uploads their descriptors (one copy per phase).
@@ -35,6 +33,8 @@ struct batch_group {
     int deg_first[4] = {0, 0, 0, 0};  // first item of degree p
     int deg_count[4] = {0, 0, 0, 0};  // items of degree p
     int deg_blocks[4][4] = {};        // element-kernel blocks of degree p in colour c
+    void* strip_items = nullptr;  // march2_item<T>[nitems], degree 3 first
+    int strip_blocks = 0;
     void* sx_items = nullptr;  // sweep_item<T>[nitems], x lines
     int sx_blocks = 0;
     void* sy_items = nullptr;  // y lines
@@ -63,7 +63,7 @@ struct adsg_batch {
     int phase = 0;
     std::vector<adsg_rhs_form> forms;
     bool prepared = false;
-    int shape = 0;  // element tile shape: 0 = 16 x 16, 1 = 8 x 8
+    int shape = 0;  // element kernel: 0 = strips in one launch, 1 = 8 x 8 tiles in colour launches
     int sweep = 0;  // 0: segmented line sweeps where every problem allows, 1: one lane per line
     std::vector<batch_group> groups[2];
     void* items = nullptr;  // the launch items of every group, one allocation
@@ -145,14 +145,18 @@ int build_groups(adsg_batch* b) {
     // the packed sweep rows come from prepare (every direction segmented, or none)
     const bool all_seg = b->packs != nullptr;
     const int P = static_cast<int>(b->sims.size());
+    std::vector<std::array<int, 3>> sizes;
+    for (const adsg_sim* h : b->sims) sizes.push_back({h->dirs[0].tab.p, h->dirs[0].tab.dofs, h->dirs[1].tab.dofs});
+    const int rows = adsg::march2_rows(sizeof(T), sizes);
     item_stage stage;
-    std::vector<std::array<size_t, 5>> offs;  // per group, in the order of b->groups[0], [1]
+    std::vector<std::array<size_t, 6>> offs;  // per group, in the order of b->groups[0], [1]
     for (int ph = 0; ph < 2; ++ph) {
         std::vector<adsg::rhs2_item<T>> ri;
         std::vector<adsg::sweep_item<T>> sx, sy;
         std::vector<adsg::seg_item<T>> gx, gy;
         batch_group g;
         std::vector<adsg::rhs2_item<T>> rdeg[4];
+        std::vector<adsg::march2_item<T>> strips[4], st;
         for (int i = 0; i < P; ++i) {
             const adsg_sim* h = b->sims[i];
             const int p = h->dirs[0].tab.p;
@@ -177,14 +181,18 @@ int build_groups(adsg_batch* b) {
             it.prm.gy = static_cast<T>(fm.grad[1]);
             it.prm.gz = static_cast<T>(fm.grad[2]);
             it.prm.reaction = static_cast<T>(fm.reaction);
-            it.prm.store = true;  // no zero fill: the first colour to reach a DOF stores
+            it.prm.store = true;  // no zero fill: the strips, or the first colour to reach a DOF, store
             int count[4];
-            adsg::rhs2_batch_tiles(b->shape, it.X.elements, it.Y.elements, it.ntx2, count);
+            adsg::rhs2_batch_tiles(it.X.elements, it.Y.elements, it.ntx2, count);
             for (int c = 0; c < 4; ++c) {
                 it.first[c] = g.deg_blocks[p][c];
                 g.deg_blocks[p][c] += count[c];
             }
             rdeg[p].push_back(it);
+            adsg::march2_item<T> si;
+            si.a = adsg::march2_problem<T>(p, rows, it.up, it.rhs, it.X, it.Y, it.prm);
+            si.p = p;
+            strips[p].push_back(si);
             const long nx = h->dirs[0].tab.dofs, ny = h->dirs[1].tab.dofs;
             adsg::sweep_item<T> xi, yi;
             xi.u = yi.u = target;
@@ -241,11 +249,17 @@ int build_groups(adsg_batch* b) {
             g.deg_count[p] = static_cast<int>(rdeg[p].size());
             ri.insert(ri.end(), rdeg[p].begin(), rdeg[p].end());
         }
+        for (int p = 3; p >= 1; --p)
+            for (auto& si : strips[p]) {
+                si.first = g.strip_blocks;
+                g.strip_blocks += static_cast<int>(adsg::march2_strips(si.a));
+                st.push_back(si);
+            }
         if (ri.empty()) continue;
         g.nitems = static_cast<int>(ri.size());
         g.seg = all_seg;
         // byte offsets of the group's item arrays, turned into device pointers below
-        offs.push_back({stage.add(ri), stage.add(sx), stage.add(sy), all_seg ? stage.add(gx) : 0,
+        offs.push_back({stage.add(ri), stage.add(st), stage.add(sx), stage.add(sy), all_seg ? stage.add(gx) : 0,
                         all_seg ? stage.add(gy) : 0});
         b->groups[ph].push_back(g);
     }
@@ -260,10 +274,11 @@ int build_groups(adsg_batch* b) {
         for (batch_group& g : gs) {
             const auto& o = offs[k++];
             g.rhs_items = base + o[0];
-            g.sx_items = base + o[1];
-            g.sy_items = base + o[2];
-            g.gx_items = g.seg ? base + o[3] : nullptr;
-            g.gy_items = g.seg ? base + o[4] : nullptr;
+            g.strip_items = base + o[1];
+            g.sx_items = base + o[2];
+            g.sy_items = base + o[3];
+            g.gx_items = g.seg ? base + o[4] : nullptr;
+            g.gy_items = g.seg ? base + o[5] : nullptr;
         }
     return ADSG_OK;
 }
@@ -272,9 +287,9 @@ int build(adsg_batch* b) {
     return b->precision == ADSG_FP32 ? build_groups<float>(b) : build_groups<double>(b);
 }
 
-// one step of every problem, starting at arena parity b->phase: the element kernels of the
-// problems of each degree in one launch per colour (the first colour to reach a DOF stores:
-// no zero fill), the x lines of every problem (every degree) in one launch, the y lines in
+// one step of every problem, starting at arena parity b->phase: the strips of every problem in
+// one launch (or 8 x 8 tiles, one launch per degree and colour: the first colour to reach a
+// DOF stores; no zero fill), the x lines of every problem (every degree) in one launch, the y lines in
 // one, and (FP32) the update: done by the segmented y sweeps as they store their lines,
 // else a pass of its own
 template <typename T>
@@ -283,9 +298,12 @@ int batch_step_impl(adsg_batch* b) {
     hipError_t e = hipSuccess;
     for (const batch_group& g : b->groups[ph]) {
         const auto* items = static_cast<const adsg::rhs2_item<T>*>(g.rhs_items);
-        for (int p = 1; p <= 3 && e == hipSuccess; ++p)
+        if (b->shape == 0)
+            e = adsg::launch_rhs2_march_batch<T>(static_cast<const adsg::march2_item<T>*>(g.strip_items), g.nitems,
+                                                 g.strip_blocks, b->stream);
+        for (int p = 1; p <= 3 && e == hipSuccess && b->shape != 0; ++p)
             for (int c = 0; c < 4 && e == hipSuccess; ++c)
-                e = adsg::launch_rhs2_batch<T>(p, b->shape, items + g.deg_first[p], g.deg_count[p], c,
+                e = adsg::launch_rhs2_batch<T>(p, items + g.deg_first[p], g.deg_count[p], c,
                                                g.deg_blocks[p][c], b->stream);
         if (e != hipSuccess) return bhip(b, e, "batch: element kernels");
         if (g.seg && b->sweep == 0)
@@ -757,7 +775,7 @@ int adsg_batch_autotune(adsg_batch* b, double* ms_out) {
     hipEvent_t e0, e1;
     (void)hipEventCreate(&e0);
     (void)hipEventCreate(&e1);
-    // every (tile shape, line grouping) pair: 16 x 16 or 8 x 8 element tiles; lines either
+    // every (element kernel, line grouping) pair: strips or 8 x 8 element tiles; lines either
     // segmented (64 lines per workgroup of nine waves) or one lane per line (64 lines per
     // one-wave workgroup)
     int best = b->shape, best_sweep = b->sweep, rc = ADSG_OK;

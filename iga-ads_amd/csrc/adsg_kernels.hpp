@@ -3,6 +3,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <array>
+#include <vector>
+
 namespace adsg {
 
 // Factors of one band matrix for the line sweeps (layout documented in adsg_setup.hpp).
@@ -146,8 +149,8 @@ struct rhs_params {
     // describes it here (defer->spill null when there is none to do)
     rhs_fixup<T>* defer = nullptr;
     // set by launch_rhs (and for batches) when the rhs start value is not used: the owners of
-    // the one-launch tiling, and the first colour to reach a DOF in the 2D colour launches,
-    // store their entries instead of adding them
+    // the one-launch tiling, the 2D strips, and the first colour to reach a DOF in the batches'
+    // colour launches, store their entries instead of adding them
     bool store = false;
     // the start value of the rhs is start_scale * start (the load vector of a source) instead
     // of what rhs holds: rhs := start_scale * start + the element sums
@@ -157,9 +160,9 @@ struct rhs_params {
 
 // variant: kernel tuning choice (0 = coefficient block held in registers, 1 = re-read from
 // LDS, ..., 5 = element columns); bits 4..7 carry the shape of variant 5, bit 8 selects one
-// launch over all tiles with a spill fix-up instead of the 2^dim parity-colour launches (2D;
-// 3D variants 0, 1, 2 and 4 with forms without a k field or a source in the kernel;
-// prm.spill set).
+// launch over all tiles with a spill fix-up instead of the 8 parity-colour launches (variants
+// 0, 1, 2 and 4 with forms without a k field or a source in the kernel; prm.spill set). 2D
+// always runs the strips of adsg_rhs2_march.hip.
 template <typename T>
 hipError_t launch_rhs(int dim, int p, const T* u_prev, T* rhs, const dev_tables<T>* dirs,
                       const rhs_params<T>& prm, int variant, hipStream_t s);
@@ -209,6 +212,40 @@ template <typename T>
 hipError_t launch_rhs3_march(int p, const T* u_prev, T* rhs, const dev_tables<T>* dirs, const rhs_params<T>& prm,
                              const int tile[3], const int nt[3], hipStream_t s);
 
+// The 2D element loop in one launch without spill entries (adsg_rhs2_march.hip): strips of
+// 64 - p DOF columns and `rows` DOF rows, one wave each. start: when set, rhs := scale * start
+// + the sums (start may be rhs).
+template <typename T>
+struct march2_args {
+    const T *up, *kfield, *start;
+    T* rhs;
+    const T *xv, *xd, *xw, *yv, *yd, *yw;  // dev_tables' val, der, wj of both directions
+    int nx, ny, ex, ey;                    // DOFs and elements
+    int ntx, rows;                         // strips per strip row, DOF rows per strip
+    T cx, cy, mass, rdt, scale;            // -dt grad, mass, dt reaction
+};
+template <typename T>
+long march2_strips(const march2_args<T>& a) {
+    return static_cast<long>(a.ntx) * ((a.ny + a.rows - 1) / a.rows);
+}
+// one problem of a batch (no k field), first = its first block; problems of the highest degree
+// first
+template <typename T>
+struct march2_item {
+    march2_args<T> a;
+    int p = 0, first = 0;
+};
+// the rows per strip for problems of (degree, DOFs in x, DOFs in y) in one launch
+int march2_rows(int bytes, const std::vector<std::array<int, 3>>& problems);
+template <typename T>
+march2_args<T> march2_problem(int p, int rows, const T* up, T* rhs, const dev_tables<T>& X, const dev_tables<T>& Y,
+                              const rhs_params<T>& prm);
+template <typename T>
+hipError_t launch_rhs2_march(int p, const T* up, T* rhs, const dev_tables<T>* dirs, const rhs_params<T>& prm,
+                             hipStream_t s);
+template <typename T>
+hipError_t launch_rhs2_march_batch(const march2_item<T>* items, int nitems, int blocks, hipStream_t s);
+
 // Batched 2D element kernels: one item per problem (degree p, no k field, no source).
 template <typename T>
 struct rhs2_item {
@@ -219,12 +256,11 @@ struct rhs2_item {
     int ntx2[4] = {0, 0, 0, 0};   // tiles of colour c per tile row
     int first[4] = {0, 0, 0, 0};  // first block of the item in colour c's launch
 };
-// tiles of each colour for tile shape 0 (16 x 16 elements) or 1 (8 x 8)
-void rhs2_batch_tiles(int shape, int elements_x, int elements_y, int ntx2[4], int count[4]);
+// tiles of 8 x 8 elements of each colour
+void rhs2_batch_tiles(int elements_x, int elements_y, int ntx2[4], int count[4]);
 // the problems of degree p in one launch per colour
 template <typename T>
-hipError_t launch_rhs2_batch(int p, int shape, const rhs2_item<T>* items, int nitems, int colour, int blocks,
-                             hipStream_t s);
+hipError_t launch_rhs2_batch(int p, const rhs2_item<T>* items, int nitems, int colour, int blocks, hipStream_t s);
 // spill values of a 2D problem in the one-launch tiling with tiles of tx x ty elements, and
 // (with off, ext) their layout as rhs_params holds it
 long rhs2_spill_layout(int p, int tx, int ty, const int elements[2], long off[8], int ext[3][2]);

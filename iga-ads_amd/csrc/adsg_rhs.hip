@@ -889,7 +889,8 @@ __device__ __forceinline__ void rhs2_flush(const T (&R)[P + 1][P + 1], double* _
 // One tile of TX x TY elements, tile t of the given parity colour (ntx2 tiles of that colour
 // per tile row), added into rhs; or (ONE) tile t of all tiles (ntx2 of them per tile row),
 // whose owned DOF-block entries go to the rhs and the others to the spill arrays of prm
-// (rhs3_put's ownership and layout, in two directions). The LDS arrays are separate
+// (rhs3_put's ownership and layout, in two directions): the batches' 8 x 8 tiles and the
+// adjoint pair; the element loop of one problem runs in strips (adsg_rhs2_march.hip). The LDS arrays are separate
 // __shared__ objects: gathered into one struct, the compiler read the tables with
 // ds_read2_b64 pairs instead of ds_read_b128 and the p = 3 batch kernel ran 1.5x slower.
 template <typename T, int P, int TX, int TY, bool KF, bool SRC, bool ONE>
@@ -1035,13 +1036,6 @@ __device__ __forceinline__ void rhs2_tile(const T* __restrict__ up, T* __restric
         }
     }
     rhs2_flush<T, P, TX, TY, ONE>(R, acc, rhs, X, Y, prm, tx, ty);
-}
-
-template <typename T, int P, int TX, int TY, bool KF, bool SRC, bool ONE>
-__global__ __launch_bounds__(TX* TY) void k_rhs2(const T* __restrict__ up, T* __restrict__ rhs,
-                                                 dev_tables<T> X, dev_tables<T> Y,
-                                                 rhs_params<T> prm, int colour, int ntx2) {
-    rhs2_tile<T, P, TX, TY, KF, SRC, ONE>(up, rhs, X, Y, prm, colour, xcd_contiguous(blockIdx.x, gridDim.x), ntx2);
 }
 
 // d/dk_b of w^T rhs(u; k) over one 2D tile (the tile of rhs2_tile for colour, t, ntx2),
@@ -1191,8 +1185,7 @@ __global__ __launch_bounds__(TX* TY) void k_adjoint2(const T* __restrict__ w, co
 
 // Many 2D problems of degree P in one launch per parity colour: block b belongs to the last
 // item whose first[colour] <= b (items in problem order), and is tile b - first[colour] of
-// it. (A one-launch form with spill arrays measured slower here: every colour launch already
-// has thousands of tiles, and the fix-up pass costs more than the colour tails it removes.)
+// it. (The other choice of batched element kernel: the strips of adsg_rhs2_march.hip.)
 template <typename T, int P, int TX>
 __global__ __launch_bounds__(TX* TX) void k_rhs2_batch(const rhs2_item<T>* __restrict__ items, int nitems,
                                                        int colour) {
@@ -1458,25 +1451,6 @@ long rhs3_one_slots(const int elements[3]) {
     return spill_layout<P>(n, nt, off, ext);
 }
 
-template <typename T, int P, bool KF, bool SRC>
-hipError_t rhs2_colours(const T* up, T* rhs, const dev_tables<T>* d, const rhs_params<T>& prm,
-                        hipStream_t s) {
-    using TL = tile<2, P>;
-    const int ntx = (d[0].elements + TL::X - 1) / TL::X;
-    const int nty = (d[1].elements + TL::Y - 1) / TL::Y;
-    for (int c = 0; c < 4; ++c) {
-        const int cx = c & 1, cy = (c >> 1) & 1;
-        const int nx2 = (ntx - cx + 1) / 2, ny2 = (nty - cy + 1) / 2;
-        const long blocks = static_cast<long>(nx2) * ny2;
-        if (blocks == 0) continue;
-        hipLaunchKernelGGL((k_rhs2<T, P, TL::X, TL::Y, KF, SRC, false>), dim3(blocks),
-                           dim3(TL::X * TL::Y), 0, s, up, rhs, d[0], d[1], prm, c, nx2);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
-}
-
 // the 2D spill arrays: array delta (1..3) has extent n[d] in the directions with delta_d = 0
 // and nt[d] P in the others; returns the total (off, ext as rhs_params holds them)
 long spill_layout2(int p, const int n[2], const int nt[2], long off[8], int ext[3][2]) {
@@ -1492,25 +1466,6 @@ long spill_layout2(int p, const int n[2], const int nt[2], long off[8], int ext[
         total += static_cast<long>(ext[0][delta & 1]) * ext[1][delta >> 1];
     }
     return total;
-}
-
-// one launch over all tiles, then the fix-up over the DOFs
-template <typename T, int P, bool KF, bool SRC>
-hipError_t rhs2_one(const T* up, T* rhs, const dev_tables<T>* d, const rhs_params<T>& prm, hipStream_t s) {
-    using TL = tile<2, P>;
-    const int ntx = (d[0].elements + TL::X - 1) / TL::X, nty = (d[1].elements + TL::Y - 1) / TL::Y;
-    const long tiles = static_cast<long>(ntx) * nty;
-    if (tiles == 0) return hipSuccess;
-    if (!prm.spill || d[0].dofs != d[0].elements + P || d[1].dofs != d[1].elements + P) return hipErrorInvalidValue;
-    rhs_params<T> q = prm;
-    const int n[2] = {d[0].dofs, d[1].dofs}, nt[2] = {ntx, nty};
-    spill_layout2(P, n, nt, q.spill_off, q.spill_ext);
-    hipLaunchKernelGGL((k_rhs2<T, P, TL::X, TL::Y, KF, SRC, true>), dim3(tiles), dim3(TL::X * TL::Y), 0, s, up, rhs,
-                       d[0], d[1], q, 0, ntx);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const int tl[3] = {TL::X, TL::Y, 1}, nt3[3] = {ntx, nty, 1}, n3[3] = {n[0], n[1], 1};
-    return finish_one(prm, q, rhs, P, tl, nt3, n3, s);
 }
 
 // the 3D k-field gradient on the tiles of tile<3, P>: one launch over all tiles and the
@@ -1625,23 +1580,23 @@ hipError_t rhs_fields(int dim, const T* up, T* rhs, const dev_tables<T>* d,
     // per-element variant
     const bool march = dim == 3 && !src && rhs3_march_fits(sizeof(T), d[0].dofs, d[1].dofs) &&
                        (!kf || rhs3_march_kfield<T>(P));
-    const bool one = (code & kRhsOneLaunch) != 0 && prm.spill &&
-                     (dim == 2 || (variant != 3 && variant != 5 && !src && (!kf || march)));
+    const bool one = dim == 3 && (code & kRhsOneLaunch) != 0 && prm.spill && variant != 3 && variant != 5 && !src &&
+                     (!kf || march);
     // 3D in one launch: the marching kernel for variant 4 and for every form with a k field,
     // which the per-element kernels take in colour launches only (70 x 50 x 61, p = 2, FP64: 34 us
     // against 154 us in eight launches and a fill)
-    const bool marched = march && one && (kf || variant == 4);
-    if (one && dim == 3 && variant == 4 && !marched) variant = P == 3 ? 2 : 1;
+    const bool marched = dim == 2 || (march && one && (kf || variant == 4));
+    if (one && variant == 4 && !marched) variant = P == 3 ? 2 : 1;
     const long n = static_cast<long>(d[0].dofs) * d[1].dofs * (dim == 3 ? d[2].dofs : 1);
     bool overwrite = (code & kRhsOverwrite) != 0;
-    if (prm.start && !marched) {  // the marching kernel adds it as it writes its block
+    if (prm.start && !marched) {  // the marching kernels add it as they write
         const hipError_t e = launch_scale<T>(rhs, prm.start, n, prm.start_scale, s);
         if (e != hipSuccess) return e;
         prm.start = nullptr;
         overwrite = false;
     }
-    // overwrite: the one launch's owners store, and so do the first colour to reach a DOF in
-    // the 2D colour launches; the 3D colour launches add into a zero fill
+    // overwrite: the one launch's owners and the 2D strips store; the colour launches add into
+    // a zero fill
     prm.store = overwrite && !prm.start && (one || dim == 2);
     if (overwrite && !one && dim != 2) {
         const hipError_t e = launch_fill<T>(rhs, n, T(0), s);
@@ -1656,16 +1611,7 @@ hipError_t rhs_fields(int dim, const T* up, T* rhs, const dev_tables<T>* d,
         if (variant == 4) return rhs3_fields<T, P, 4>(up, rhs, d, prm, one, s);
         return rhs3_fields<T, P, 0>(up, rhs, d, prm, one, s);
     }
-    if (one) {
-        if (kf && src) return rhs2_one<T, P, true, true>(up, rhs, d, prm, s);
-        if (kf) return rhs2_one<T, P, true, false>(up, rhs, d, prm, s);
-        if (src) return rhs2_one<T, P, false, true>(up, rhs, d, prm, s);
-        return rhs2_one<T, P, false, false>(up, rhs, d, prm, s);
-    }
-    if (kf && src) return rhs2_colours<T, P, true, true>(up, rhs, d, prm, s);
-    if (kf) return rhs2_colours<T, P, true, false>(up, rhs, d, prm, s);
-    if (src) return rhs2_colours<T, P, false, true>(up, rhs, d, prm, s);
-    return rhs2_colours<T, P, false, false>(up, rhs, d, prm, s);
+    return launch_rhs2_march<T>(P, up, rhs, d, prm, s);
 }
 
 }  // namespace
@@ -1790,9 +1736,8 @@ long rhs_spill_slots(int dim, int p, const int elements[3]) {
     }
 }
 
-void rhs2_batch_tiles(int shape, int elements_x, int elements_y, int ntx2[4], int count[4]) {
-    const int TX = shape == 0 ? 16 : 8, TY = TX;
-    const int ntx = (elements_x + TX - 1) / TX, nty = (elements_y + TY - 1) / TY;
+void rhs2_batch_tiles(int elements_x, int elements_y, int ntx2[4], int count[4]) {
+    const int ntx = (elements_x + 7) / 8, nty = (elements_y + 7) / 8;
     for (int c = 0; c < 4; ++c) {
         const int cx = c & 1, cy = (c >> 1) & 1;
         ntx2[c] = (ntx - cx + 1) / 2;
@@ -1801,23 +1746,17 @@ void rhs2_batch_tiles(int shape, int elements_x, int elements_y, int ntx2[4], in
 }
 
 template <typename T>
-hipError_t launch_rhs2_batch(int p, int shape, const rhs2_item<T>* items, int nitems, int colour, int blocks,
-                             hipStream_t s) {
+hipError_t launch_rhs2_batch(int p, const rhs2_item<T>* items, int nitems, int colour, int blocks, hipStream_t s) {
     if (blocks <= 0 || nitems <= 0) return hipSuccess;
-#define ADSG_RB(P_, TX_)                                                                                  \
-    if (p == P_ && TX_ == (shape == 0 ? 16 : 8)) {                                                        \
-        hipLaunchKernelGGL((k_rhs2_batch<T, P_, TX_>), dim3(blocks), dim3(TX_ * TX_), 0, s, items, nitems, \
-                           colour);                                                                       \
-        return hipGetLastError();                                                                         \
-    }
-    ADSG_RB(1, 16)
-    ADSG_RB(2, 16)
-    ADSG_RB(3, 16)
-    ADSG_RB(1, 8)
-    ADSG_RB(2, 8)
-    ADSG_RB(3, 8)
-#undef ADSG_RB
-    return hipErrorInvalidValue;
+    if (p == 1)
+        hipLaunchKernelGGL((k_rhs2_batch<T, 1, 8>), dim3(blocks), dim3(64), 0, s, items, nitems, colour);
+    else if (p == 2)
+        hipLaunchKernelGGL((k_rhs2_batch<T, 2, 8>), dim3(blocks), dim3(64), 0, s, items, nitems, colour);
+    else if (p == 3)
+        hipLaunchKernelGGL((k_rhs2_batch<T, 3, 8>), dim3(blocks), dim3(64), 0, s, items, nitems, colour);
+    else
+        return hipErrorInvalidValue;
+    return hipGetLastError();
 }
 
 template hipError_t launch_kgrad<double>(int, int, const double*, const double*, double*, const dev_tables<double>*,
@@ -1827,8 +1766,8 @@ template hipError_t launch_adjoint2<double>(int, const double*, const double*, d
                                             const rhs_params<double>&, double*, double*, hipStream_t);
 template hipError_t launch_rhs_fixup<double>(double*, const rhs_fixup<double>&, hipStream_t);
 template hipError_t launch_rhs_fixup<float>(float*, const rhs_fixup<float>&, hipStream_t);
-template hipError_t launch_rhs2_batch<double>(int, int, const rhs2_item<double>*, int, int, int, hipStream_t);
-template hipError_t launch_rhs2_batch<float>(int, int, const rhs2_item<float>*, int, int, int, hipStream_t);
+template hipError_t launch_rhs2_batch<double>(int, const rhs2_item<double>*, int, int, int, hipStream_t);
+template hipError_t launch_rhs2_batch<float>(int, const rhs2_item<float>*, int, int, int, hipStream_t);
 template hipError_t launch_rhs<double>(int, int, const double*, double*, const dev_tables<double>*,
                                        const rhs_params<double>&, int, hipStream_t);
 template hipError_t launch_rhs<float>(int, int, const float*, float*, const dev_tables<float>*,

@@ -295,7 +295,7 @@ int adsg_check_finite(adsg_sim* h, int which);
  * slots is NULL, adsg_step_delta's with these slots otherwise -- measured with HIP events on
  * the handle's stream: the counterpart of the reference's StatTimer around compute_rhs
  * (examples/scalability/test3d.hpp:67-101). Averages per step in milliseconds: ms[0] the
- * element-loop kernels (the 2^dim colour launches, or the one launch over all tiles),
+ * element-loop kernels (the colour launches, or the one launch over all tiles),
  * ms[1] boundary handling, ms[2], ms[3], ms[4] line sweeps in x, y, z, ms[5] the whole step,
  * ms[6] the start of the rhs (a source's load vector scaled in; the zero fill, where one is
  * needed, is part of ms[0]). With the one-launch tiling the spill fix-up, and the FP64
@@ -337,15 +337,15 @@ int adsg_time_phases(adsg_sim* h, int nsteps, const adsg_rhs_form* form, const i
  * of elements along z, the x-y contractions on the matrix cores): bit 0 two columns per
  * wave, bit 1 three chunks of 16 DOF planes per workgroup; the autotuner times all four. */
 #define ADSG_TUNE_RHS_COLUMNS 4
-/* ADSG_TUNE_RHS_TILING (2D every form; 3D variants 0, 1, 2 and 4; forms with a k field run
- * variant 4's kernel then, in FP32 for p <= 2): 0 = 2^dim parity-colour launches, whose tiles share no
- * DOF; 1 = one launch over all tiles, each tile adding the entries of its DOF block that it
+/* ADSG_TUNE_RHS_TILING (3D variants 0, 1, 2 and 4; forms with a k field run variant 4's
+ * kernel then, in FP32 for p <= 2): 0 = 8 parity-colour launches, whose tiles share no DOF; 1 = one launch over all tiles, each tile adding the entries of its DOF block that it
  * owns and storing the others in a spill array (allocated with the handle, about one to
  * three values per element), which a second kernel adds in a fixed order. Both are
- * deterministic; the sums are grouped differently (equal to rounding). Default 1 in 3D and
- * for 2D meshes of at most 2048 tiles of 16 x 16 elements, 0 for larger 2D meshes (and in
- * batches, whose problems therefore equal the same problems run alone with 0). The
- * autotuner times both. */
+ * deterministic; the sums are grouped differently (equal to rounding). The autotuner times
+ * both. The 2D element loop is one launch of strips that share no DOF with either value (and
+ * in batches, whose problems therefore equal the same problems run alone); there the tiling is
+ * that of the k-field gradients. Default 1 in 3D and for 2D meshes of at most 2048 tiles of
+ * 16 x 16 elements, 0 for larger 2D meshes. */
 #define ADSG_TUNE_RHS_TILING 5
 /* ADSG_TUNE_CACHE (default 1): adsg_autotune records its choices per configuration (device,
  * dimension, precision, degree / elements / Gauss points / repeated nodes per direction, the
@@ -363,8 +363,8 @@ int adsg_autotune(adsg_sim* h, const adsg_rhs_form* form, const int* slots, int 
  * validation.hpp:73-81) with natural boundaries, its own mesh size and degree p = 1..3 (the
  * same in x and y), and a form without k field or source (e.g. the reaction-diffusion form
  * {mass 1, dt, grad eps, reaction 1}). The state of all problems lives in shared arenas;
- * one step is a fixed sequence of grouped launches over all problems (element kernels per
- * degree and colour, x and y sweeps per degree, one update), and nsteps steps are replayed
+ * one step is a fixed sequence of grouped launches over all problems (one element kernel, x
+ * and y sweeps, the update), and nsteps steps are replayed
  * from HIP graphs of at most 50 steps, each captured once per step count. FP32 batches use
  * the increment scheme of ADSG_FP32. The set-up runs on the device: adsg_batch_create
  * tabulates every problem's basis (basis_data.cpp:63-114) in one launch, adsg_batch_prepare
@@ -390,12 +390,13 @@ int adsg_batch_set_vector(adsg_batch* b, int problem, int which, const double* h
 int adsg_batch_get_vector(adsg_batch* b, int problem, int which, double* host);
 int adsg_batch_step(adsg_batch* b, int nsteps);
 int adsg_batch_synchronize(adsg_batch* b);
-/* ADSG_TUNE_BATCH_TILE: element tile of the batched kernels, 0 = 16 x 16, 1 = 8 x 8.
+/* ADSG_TUNE_BATCH_TILE: element kernel of the batch, 0 = strips of every problem in one
+ * launch, 1 = tiles of 8 x 8 elements, one launch per degree and parity colour.
  * ADSG_TUNE_SWEEP_VARIANT: 0 = segmented line sweeps (9 waves per 64 lines; used when every
  * problem's lines split into segments), 1 = one lane per line.
- * adsg_batch_autotune times one step with each tile shape and each line grouping (the two
+ * adsg_batch_autotune times one step with each element kernel and each line grouping (the two
  * sweep variants), keeps the fastest pair and restores the state; ms_out[0..1] (may be
- * NULL) receives each tile shape's time with its better sweep variant. */
+ * NULL) receives each element kernel's time with its better sweep variant. */
 #define ADSG_TUNE_BATCH_TILE 2
 int adsg_batch_set_tuning(adsg_batch* b, int key, int value);
 int adsg_batch_get_tuning(const adsg_batch* b, int key);
