@@ -225,7 +225,7 @@ int build_groups(adsg_batch* b) {
                 a.nseg = sgx.nseg;
                 a.p = p;
                 a.first = g.gx_blocks;
-                g.gx_blocks += static_cast<int>((ny + 63) / 64);
+                g.gx_blocks += static_cast<int>((ny + adsg::seg_batch_lines(a.nseg) - 1) / adsg::seg_batch_lines(a.nseg));
                 c.g = yi.g;
                 if constexpr (sizeof(T) == sizeof(float)) {  // the y sweep does the FP32 step's update
                     c.x_prev = b->u[ph] + b->off[i];
@@ -238,7 +238,7 @@ int build_groups(adsg_batch* b) {
                 c.nseg = sgy.nseg;
                 c.p = p;
                 c.first = g.gy_blocks;
-                g.gy_blocks += static_cast<int>((nx + 63) / 64);
+                g.gy_blocks += static_cast<int>((nx + adsg::seg_batch_lines(c.nseg) - 1) / adsg::seg_batch_lines(c.nseg));
                 gx.push_back(a);
                 gy.push_back(c);
             }
@@ -308,14 +308,14 @@ int batch_step_impl(adsg_batch* b) {
         if (e != hipSuccess) return bhip(b, e, "batch: element kernels");
         if (g.seg && b->sweep == 0)
             e = adsg::launch_sweep_seg_batch<T>(static_cast<const adsg::seg_item<T>*>(g.gx_items), g.nitems,
-                                                g.gx_blocks, b->stream);
+                                                g.gx_blocks, true, b->stream);
         else
             e = adsg::launch_sweep_batch<T>(static_cast<const adsg::sweep_item<T>*>(g.sx_items), g.nitems,
                                             g.sx_blocks, b->stream);
         if (e != hipSuccess) return bhip(b, e, "batch: x sweeps");
         if (g.seg && b->sweep == 0)
             e = adsg::launch_sweep_seg_batch<T>(static_cast<const adsg::seg_item<T>*>(g.gy_items), g.nitems,
-                                                g.gy_blocks, b->stream);
+                                                g.gy_blocks, false, b->stream);
         else
             e = adsg::launch_sweep_batch<T>(static_cast<const adsg::sweep_item<T>*>(g.sy_items), g.nitems,
                                             g.sy_blocks, b->stream);

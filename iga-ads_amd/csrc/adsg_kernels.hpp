@@ -280,9 +280,11 @@ hipError_t launch_sweep_batch(const sweep_item<T>* items, int nitems, int blocks
 
 // Batched segmented sweeps (unpivoted factors): one item per (problem, direction) with its
 // packed rows (line_segments::pack, segmented for at most kBatchSegments segments of at
-// most 32 rows), problems of every degree p in one launch, 64 lines per block of
-// kBatchSegments waves; first = first block of the item.
+// most 32 rows), problems of every degree p in one launch, seg_batch_lines lines per block of
+// kBatchSegments waves; first = first block of the item. All items of a launch are x lines
+// (g.S == 1, consecutive) or strided ones.
 constexpr int kBatchSegments = 9;
+constexpr int seg_batch_lines(int nseg) { return 64 * (kBatchSegments / nseg); }
 template <typename T>
 struct seg_item {
     T* u = nullptr;
@@ -297,7 +299,7 @@ struct seg_item {
     float* shadow = nullptr;
 };
 template <typename T>
-hipError_t launch_sweep_seg_batch(const seg_item<T>* items, int nitems, int blocks, hipStream_t s);
+hipError_t launch_sweep_seg_batch(const seg_item<T>* items, int nitems, int blocks, bool x_lines, hipStream_t s);
 
 // d/dk of w^T rhs(u; k) for the gradient term of prm, added into out:
 //   out_b += -dt sum_e sum_q w_q J_e B_b(x_q) sum_d grad_d (d_d u)(d_d w)
