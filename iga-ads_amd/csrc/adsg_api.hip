@@ -122,20 +122,31 @@ int upload_tables(adsg_sim* h, dev_dir& d) {
         const size_t a = i % (d.tab.p + 1), r = i / (d.tab.p + 1), k = (r / 4) * (d.tab.p + 1) + a;
         pack[i] = r % 4 == 0 ? val[k] : r % 4 == 1 ? der[k] : r % 4 == 2 ? bval[k] : bder[k];
     }
-    if (h->dim == 3 && (rc = h->precision == ADSG_FP32 ? upload<float>(h, &d.pack, pack) : upload<double>(h, &d.pack, pack)))
-        return rc;
-    if (h->precision == ADSG_FP32) {
-        if ((rc = upload<float>(h, &d.val, val))) return rc;
-        if ((rc = upload<float>(h, &d.der, der))) return rc;
-        if ((rc = upload<float>(h, &d.bval, bval))) return rc;
-        if ((rc = upload<float>(h, &d.bder, bder))) return rc;
-        if ((rc = upload<float>(h, &d.wj, d.tab.wj))) return rc;
-    } else {
-        if ((rc = upload<double>(h, &d.val, val))) return rc;
-        if ((rc = upload<double>(h, &d.der, der))) return rc;
-        if ((rc = upload<double>(h, &d.bval, bval))) return rc;
-        if ((rc = upload<double>(h, &d.bder, bder))) return rc;
-        if ((rc = upload<double>(h, &d.wj, d.tab.wj))) return rc;
+    // one allocation and one copy for the direction's tables
+    struct table {
+        void** to;
+        const std::vector<double>* from;
+    };
+    const table tables[] = {{&d.val, &val}, {&d.der, &der}, {&d.bval, &bval}, {&d.bder, &bder}, {&d.wj, &d.tab.wj}, {&d.pack, &pack}};
+    const size_t unit = h->precision == ADSG_FP32 ? sizeof(float) : sizeof(double);
+    auto bytes = [&](const table& t) { return (t.from->size() * unit + 255) / 256 * 256; };
+    size_t total = 0;
+    for (const table& t : tables) total += bytes(t);
+    std::vector<char> host(std::max<size_t>(total, 256));
+    size_t at = 0;
+    for (const table& t : tables) {
+        for (size_t i = 0; i < t.from->size(); ++i)
+            if (unit == sizeof(float))
+                reinterpret_cast<float*>(host.data() + at)[i] = static_cast<float>((*t.from)[i]);
+            else
+                reinterpret_cast<double*>(host.data() + at)[i] = (*t.from)[i];
+        at += bytes(t);
+    }
+    if ((rc = upload_bytes(h, &d.tables, host.data(), host.size()))) return rc;
+    at = 0;
+    for (const table& t : tables) {
+        *t.to = t.from->empty() ? nullptr : static_cast<char*>(d.tables) + at;
+        at += bytes(t);
     }
     // form_matrix.cpp:8-42 on the same tables: the Gram and stiffness matrices, unfixed, in
     // FP64 in both precisions (the separable rhs contracts in FP64)
@@ -1127,7 +1138,7 @@ void adsg_destroy(adsg_sim* h) {
     drop_graphs(h);
     for (auto& d : h->dirs) {
         for (auto& s : d.slots) free_slot(s, h->in_arena);
-        for (void** p : {&d.val, &d.der, &d.wj, &d.bval, &d.bder, &d.pack, &d.rows, &d.kM, &d.kK})
+        for (void** p : {&d.tables, &d.rows, &d.kM, &d.kK})
             if (*p && !h->in_arena) (void)hipFree(*p);
         if (d.first && !h->in_arena) (void)hipFree(d.first);
     }

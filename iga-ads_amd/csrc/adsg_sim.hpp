@@ -44,7 +44,8 @@ struct dev_dir {
     void* wj = nullptr;
     void* bval = nullptr;  // val, der times the Gauss weight (padded like val)
     void* bder = nullptr;
-    void* pack = nullptr;  // val, der, bval, bder of an element together (dev_tables::pack)
+    void* pack = nullptr;  // val, der, bval, bder of an element together (dev_tables::pack; 3D)
+    void* tables = nullptr;  // the allocation that holds them (none in a batch's arena)
     void* rows = nullptr;  // FP32 mode: slot-0 matrix as n rows of 2p+1 entries
     // the 1D Gram and stiffness matrices as rows of 2p+1 entries (step precision), for the
     // separable-integrand rhs (launch_rhs_kron)
