@@ -288,7 +288,8 @@ int sweep_dir(adsg_sim* h, T* u, int d, int sl, int mode = 0, const adsg::rhs_fi
     f.kl = s.lf.kl;
     f.ku = s.lf.ku_eff;
     f.pivoted = s.lf.pivoted;
-    const bool seg_ok = s.seg.nseg > 0;
+    // lines of one segment (up to 16 rows): the plain solve only
+    const bool seg_ok = s.seg.nseg > (mode == 0 ? 0 : 1);
     if (mode != 0 && !seg_ok)
         return fail(h, ADSG_EINVAL,
                     "ads_solve: transposed and refined solves need unpivoted factors and lines of "

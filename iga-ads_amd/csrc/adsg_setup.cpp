@@ -287,7 +287,7 @@ int factor_for_lines(const std::vector<double>& ab_in, int n, int kl, int ku, li
     return info;
 }
 
-bool segment_shape(int n, int km, int max_nseg16, int max_nseg32, int& m, int& nseg, int& mseg) {
+bool segment_shape(int n, int km, int max_nseg16, int max_nseg32, int& m, int& nseg, int& mseg, int min_nseg) {
     mseg = nseg = m = 0;
     // the fewest segments of at most `rows` rows (balanced lengths, the last one at least km
     // rows long) within the caller's count limit: the serial chain between segments costs
@@ -296,7 +296,7 @@ bool segment_shape(int n, int km, int max_nseg16, int max_nseg32, int& m, int& n
     auto pick = [&](int max_s, int rows) {
         if (mseg) return;
         const int s = (n + rows - 1) / rows;
-        if (s < 2 || s > max_s) return;
+        if (s < min_nseg || s > max_s) return;
         const int mm = (n + s - 1) / s;
         if (mm > rows || mm < km || n - (s - 1) * mm < km) return;
         mseg = rows;
@@ -313,7 +313,7 @@ bool segment_lines(const line_factors& f, line_segments& out, int max_nseg16, in
     const int km = std::max(kl, ku);
     if (f.pivoted || kl < 1 || ku < 1 || kl != ku) return false;
     int mseg = 0, nseg = 0, m = 0;
-    if (!segment_shape(n, km, max_nseg16, max_nseg32, m, nseg, mseg)) return false;
+    if (!segment_shape(n, km, max_nseg16, max_nseg32, m, nseg, mseg, 1)) return false;
     out.m = m;
     out.nseg = nseg;
     out.mseg = mseg;

@@ -82,7 +82,9 @@ struct line_segments {
 // <= 32 rows if <= max_nseg32 (the callers' limits keep the kernels' LDS within budget).
 bool segment_lines(const line_factors& f, line_segments& out, int max_nseg16, int max_nseg32);
 // The segment shape segment_lines picks for lines of n rows with half-bandwidth km:
-// m rows per segment, nseg segments in blocks of mseg rows; false when none fits.
-bool segment_shape(int n, int km, int max_nseg16, int max_nseg32, int& m, int& nseg, int& mseg);
+// m rows per segment, nseg >= min_nseg segments in blocks of mseg rows; false when none fits.
+// (segment_lines: from one segment on, lines of up to 16 rows, which one lane per line solved in
+// 15.4 / 9.3 / 9.3 us at 11 x 12 x 14 and the segmented sweep in 6.5 / 6.6 / 6.3.)
+bool segment_shape(int n, int km, int max_nseg16, int max_nseg32, int& m, int& nseg, int& mseg, int min_nseg = 2);
 
 }  // namespace adsg

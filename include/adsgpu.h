@@ -318,7 +318,7 @@ int adsg_time_phases(adsg_sim* h, int nsteps, const adsg_rhs_form* form, const i
  * at p = 2 in FP64 and 2^20 otherwise; below, 2 for FP64 p = 3 and else 1).
  * ADSG_TUNE_SWEEP_VARIANT selects the line sweep (0: lines cut into segments solved by
  * separate waves and joined through FP64-computed influence coefficients, where the factors
- * are unpivoted and the lines are 2..16 segments of at most 32 rows long (up to 512 DOFs),
+ * are unpivoted and the lines are 1..16 segments of at most 32 rows long (up to 512 DOFs),
  * x lines staged through LDS where that fits; 1: one lane per whole line; 2: as 0 with the x
  * lines read lane by lane, faster on some small meshes).
  * adsg_autotune times every variant on the handle's current state with the given form

@@ -56,3 +56,17 @@ def test_fp32_increments_at_segment_edges_match_oracle(p):
         r = o.compute_rhs(u, po.heat_form(dt, 2))
         assert po.rel_l2(g.get(ag.U) - u, o.solve(r) - u) <= bound, (nx, ny)
         g.close()
+
+
+@pytest.mark.parametrize("p", [1, 2, 3])
+def test_one_segment_lines_match_oracle_and_transposed_stays_refused(p):
+    """Lines of at most 16 DOFs: one segment, the plain solve only."""
+    for nx, ny in [(p + 1, p + 1), (p + 2, 16), (15, 17), (16, 40), (16, p + 1)]:
+        g, o = _pair(p, nx, ny, ag.FP64)
+        b = np.random.default_rng(nx + ny + p).standard_normal(g.size)
+        g.set(ag.U, b)
+        g.ads_solve()
+        assert po.rel_l2(g.get(ag.U), o.solve(b.copy())) <= 1e-13, (nx, ny)
+        with pytest.raises(ag.AdsgError):
+            g.ads_solve_transposed()
+        g.close()
