@@ -131,12 +131,12 @@ struct dev_tables {
 };
 
 // Integrand of compute_rhs at a Gauss point:
-//   mass*u*v - dt*k*(gx*ux*vx + gy*uy*vy + gz*uz*vz) + dt*reaction*u*(1-u)*v + dt*f*v
+//   mass*u*v - dt*k*(gx*ux*vx + gy*uy*vy + gz*uz*vz) + dt*reaction*u*(1-u)*v
+// (a source's dt*f*v enters as the start value)
 template <typename T>
 struct rhs_params {
     T mass = 1, dt = 0, gx = 1, gy = 1, gz = 1, reaction = 0;
     const T* kfield = nullptr;  // coefficients of k on the same basis, or null (k = 1)
-    const T* source = nullptr;  // coefficients of f on the same basis, or null (f = 0)
     // one-launch tiling (element-kernel code bit 8): rhs_spill_slots(dim, p, elements) values
     // for the block entries a tile does not own; null selects the colour launches. The
     // entries go to 7 arrays, one per neighbour offset delta = dx + 2 dy + 4 dz (1..7) of the
@@ -161,7 +161,7 @@ struct rhs_params {
 // variant: kernel tuning choice (0 = coefficient block held in registers, 1 = re-read from
 // LDS, ..., 5 = element columns); bits 4..7 carry the shape of variant 5, bit 8 selects one
 // launch over all tiles with a spill fix-up instead of the 8 parity-colour launches (variants
-// 0, 1, 2 and 4 with forms without a k field or a source in the kernel; prm.spill set). 2D
+// 0, 1, 2 and 4 with forms without a k field; prm.spill set). 2D
 // always runs the strips of adsg_rhs2_march.hip.
 template <typename T>
 hipError_t launch_rhs(int dim, int p, const T* u_prev, T* rhs, const dev_tables<T>* dirs,
@@ -184,7 +184,7 @@ template <typename T>
 hipError_t launch_rhs_general(int dim, const T* u_prev, T* rhs, const dev_tables<T>* dirs, const rhs_params<T>& prm,
                               hipStream_t s);
 
-// Variant 5 (3D, p = 2 or 3, forms without a k field or a source in the kernel): element
+// Variant 5 (3D, p = 2 or 3, forms without a k field): element
 // columns with the x-y contractions on the matrix cores (adsg_rhs_col.hip); shape 0..3
 // selects columns per wave (bit 0: two) and chunks per z-range (bit 1: three).
 template <typename T>
@@ -195,7 +195,7 @@ hipError_t launch_rhs3_col(int p, const T* u_prev, T* rhs, const dev_tables<T>* 
 
 // Variant 4 in one launch (adsg_rhs_march.hip): its tiles (elements per tile and tile counts
 // per direction) for degree p, values of `bytes` bytes, with or without a k field; and its
-// launch on them (prm: the spill layout of these tiles set; no source in the kernel).
+// launch on them (prm: the spill layout of these tiles set).
 // Forms with a k field: not FP32 at p = 3, where the sums along z in FP32 were 10 to 22 % further
 // from FP64 than the per-element kernels' sums across elements in FP64 (10 heat steps, 64^3 and
 // 128 x 100 x 90); everywhere else its FP32 error is no larger than theirs.

@@ -114,13 +114,12 @@ __device__ __forceinline__ void rhs3_put(const block_sink<T>& k, const rhs_param
 // of its elements: xt[FV], xt[FD] as tabulated, xt[BV], xt[BD] with the quadrature weight
 // (variants 0-2 also fold -dt*grad_x into xt[BD], -dt*grad_y into yt[BD]).
 enum { FV = 0, FD = 1, BV = 2, BD = 3 };
-template <typename T, int P, int TX, int TY, int TZ, bool KF, bool SRC>
+template <typename T, int P, int TX, int TY, int TZ, bool KF>
 struct rhs3_buf {
     static constexpr int M = P + 1, BX = TX + P, BY = TY + P, BZ = TZ + P;
     static constexpr int NB = BX * BY * BZ, PL = BX * BY;
     T blk[NB];
     T kb[KF ? NB : 1];
-    T sb[SRC ? NB : 1];
     T xt[4][TX * M * M];
     T yt[4][TY * M * M];
 };
@@ -133,9 +132,9 @@ constexpr int rhs3_acc_size() {
 // The LDS of a workgroup with NBUF tile buffers and their planes, in one object: the
 // compiler then addresses every part from one base (separate __shared__ arrays cost
 // registers in the element loop).
-template <typename T, int P, int TX, int TY, int TZ, bool KF, bool SRC, int NBUF>
+template <typename T, int P, int TX, int TY, int TZ, bool KF, int NBUF>
 struct rhs3_lds {
-    rhs3_buf<T, P, TX, TY, TZ, KF, SRC> b[NBUF];
+    rhs3_buf<T, P, TX, TY, TZ, KF> b[NBUF];
     double acc[NBUF][rhs3_acc_size<P, TX, TY, TZ>()];
 };
 
@@ -143,23 +142,23 @@ struct rhs3_lds {
 // sum-factorised integrand over its Gauss points, its contribution accumulated in R (owned
 // and zeroed by the caller) and added to the wave's planes, or (variant 4) left in R for
 // the caller, which carries the planes shared with the wave's next element layer.
-template <typename T, int P, int TX, int TY, int TZ, bool KF, bool SRC, int FM, int VAR>
-__device__ __forceinline__ void rhs3_element(const rhs3_buf<T, P, TX, TY, TZ, KF, SRC>& L,
+template <typename T, int P, int TX, int TY, int TZ, bool KF, int FM, int VAR>
+__device__ __forceinline__ void rhs3_element(const rhs3_buf<T, P, TX, TY, TZ, KF>& L,
                                              double* acc, const dev_tables<T>& X,
                                              const dev_tables<T>& Y, const dev_tables<T>& Z,
                                              const rhs_params<T>& prm, int lx, int ly, int lz,
                                              int ex0, int ey0, int ez0,
                                              T (&R)[P + 1][P + 1][P + 1]) {
-    using LDS = rhs3_buf<T, P, TX, TY, TZ, KF, SRC>;
+    using LDS = rhs3_buf<T, P, TX, TY, TZ, KF>;
     constexpr int M = P + 1, BX = LDS::BX, BY = LDS::BY, PL = LDS::PL;
     constexpr bool CREG = VAR == 0;  // coefficient block held in registers
     // element contribution added to the planes per x point (variant 3 at P = 3: registers)
     constexpr bool FLUSH = VAR == 2 || (VAR == 3 && P == 3);
     constexpr bool TW = VAR == 3;  // tables weighted only: -dt*grad applied as read
     // FM: 0 the heat form (mass term), 1 with the reaction term, 2 no mass term (mass = 0, no
-    // reaction, no source: the delta and FP32 increment forms), where u itself is not needed
+    // reaction: the delta and FP32 increment forms), where u itself is not needed
     constexpr bool RX = FM == 1, MS = FM != 2;
-    static_assert(MS || (!SRC && !RX), "form 2 has no term in v other than the gradient terms");
+    static_assert(MS || !RX, "form 2 has no term in v other than the gradient terms");
     static_assert(VAR != 4 || P <= 2, "variant 4 carries the register block: p <= 2");
     const int ez = ez0 + lz;
     // the wave's planes: in one add instruction the 64 lanes hit 64 distinct entries
@@ -184,18 +183,16 @@ __device__ __forceinline__ void rhs3_element(const rhs3_buf<T, P, TX, TY, TZ, KF
         const T cz = -prm.dt * prm.gz;
         const T cx = -prm.dt * prm.gx, cy = -prm.dt * prm.gy;  // used by TW only
         // per z point constants with the weight folded in (wave-uniform)
-        T mwz[M], cwz[M], swz[M], rwz[M];
+        T mwz[M], cwz[M], rwz[M];
 #pragma unroll
         for (int q = 0; q < M; ++q) {
             mwz[q] = prm.mass * wz[q];
             cwz[q] = cz * wz[q];
-            swz[q] = prm.dt * wz[q];
             rwz[q] = prm.dt * prm.reaction * wz[q];
         }
         if (ex0 + lx < X.elements && ey0 + ly < Y.elements) {
             T cf[CREG ? M : 1][CREG ? M : 1][CREG ? M : 1];
             T kc[KF && CREG ? M : 1][KF && CREG ? M : 1][KF && CREG ? M : 1];
-            T sc[SRC && CREG ? M : 1][SRC && CREG ? M : 1][SRC && CREG ? M : 1];
             if constexpr (CREG) {
 #pragma unroll
                 for (int a = 0; a < M; ++a)
@@ -206,7 +203,6 @@ __device__ __forceinline__ void rhs3_element(const rhs3_buf<T, P, TX, TY, TZ, KF
                             const int li = (lx + a) + BX * ((ly + b) + BY * (lz + c));
                             cf[a][b][c] = L.blk[li];
                             if constexpr (KF) kc[a][b][c] = L.kb[li];
-                            if constexpr (SRC) sc[a][b][c] = L.sb[li];
                         }
             }
 #pragma unroll 1
@@ -218,12 +214,12 @@ __device__ __forceinline__ void rhs3_element(const rhs3_buf<T, P, TX, TY, TZ, KF
                     dx[a] = L.xt[FD][(lx * M + qx) * M + a];
                 }
                 // stage x: contract the element's first index
-                T A0[M][M], A1[M][M], KA[KF ? M : 1][KF ? M : 1], SA[SRC ? M : 1][SRC ? M : 1];
+                T A0[M][M], A1[M][M], KA[KF ? M : 1][KF ? M : 1];
 #pragma unroll
                 for (int b = 0; b < M; ++b)
 #pragma unroll
                     for (int c = 0; c < M; ++c) {
-                        T s0 = 0, s1 = 0, sk = 0, ss = 0;
+                        T s0 = 0, s1 = 0, sk = 0;
 #pragma unroll
                         for (int a = 0; a < M; ++a) {
                             const int li = (lx + a) + BX * ((ly + b) + BY * (lz + c));
@@ -232,13 +228,10 @@ __device__ __forceinline__ void rhs3_element(const rhs3_buf<T, P, TX, TY, TZ, KF
                             s1 += dx[a] * cv;
                             if constexpr (KF)
                                 sk += bx[a] * (CREG ? kc[KF && CREG ? a : 0][KF && CREG ? b : 0][KF && CREG ? c : 0] : L.kb[li]);
-                            if constexpr (SRC)
-                                ss += bx[a] * (CREG ? sc[SRC && CREG ? a : 0][SRC && CREG ? b : 0][SRC && CREG ? c : 0] : L.sb[li]);
                         }
                         A0[b][c] = s0;
                         A1[b][c] = s1;
                         if constexpr (KF) KA[b][c] = sk;
-                        if constexpr (SRC) SA[b][c] = ss;
                     }
                 T K0[M][M], Kx[M][M];
 #pragma unroll
@@ -254,23 +247,21 @@ __device__ __forceinline__ void rhs3_element(const rhs3_buf<T, P, TX, TY, TZ, KF
                         dy[b] = L.yt[FD][(ly * M + qy) * M + b];
                     }
                     // stage y for this Gauss point
-                    T a00[M], a01[M], a10[M], ka[KF ? M : 1], sa[SRC ? M : 1];
+                    T a00[M], a01[M], a10[M], ka[KF ? M : 1];
 #pragma unroll
                     for (int c = 0; c < M; ++c) {
-                        T s00 = 0, s01 = 0, s10 = 0, sk = 0, ss = 0;
+                        T s00 = 0, s01 = 0, s10 = 0, sk = 0;
 #pragma unroll
                         for (int b = 0; b < M; ++b) {
                             s00 += by[b] * A0[b][c];
                             s01 += dy[b] * A0[b][c];
                             s10 += by[b] * A1[b][c];
                             if constexpr (KF) sk += by[b] * KA[b][c];
-                            if constexpr (SRC) ss += by[b] * SA[b][c];
                         }
                         a00[c] = s00;
                         a01[c] = s01;
                         a10[c] = s10;
                         if constexpr (KF) ka[c] = sk;
-                        if constexpr (SRC) sa[c] = ss;
                     }
                     T H0[M], Hx[M], Hy[M];
 #pragma unroll
@@ -278,7 +269,7 @@ __device__ __forceinline__ void rhs3_element(const rhs3_buf<T, P, TX, TY, TZ, KF
 #pragma unroll
                     for (int qz = 0; qz < M; ++qz) {
                         // stage z, the integrand, and stage z transposed
-                        T u = 0, uz = 0, uy = 0, ux = 0, kv = 0, fv = 0;
+                        T u = 0, uz = 0, uy = 0, ux = 0, kv = 0;
 #pragma unroll
                         for (int c = 0; c < M; ++c) {
                             if constexpr (MS) u += Bz[qz][c] * a00[c];
@@ -286,11 +277,9 @@ __device__ __forceinline__ void rhs3_element(const rhs3_buf<T, P, TX, TY, TZ, KF
                             uy += Bz[qz][c] * a01[c];
                             ux += Bz[qz][c] * a10[c];
                             if constexpr (KF) kv += Bz[qz][c] * ka[c];
-                            if constexpr (SRC) fv += Bz[qz][c] * sa[c];
                         }
                         T g0 = MS ? mwz[qz] * u : T(0);
                         if constexpr (RX) g0 += rwz[qz] * u * (T(1) - u);
-                        if constexpr (SRC) g0 += swz[qz] * fv;
                         T gx, gy, gz;
                         if constexpr (KF) {
                             const T kw = wz[qz] * kv;
@@ -361,12 +350,12 @@ __device__ __forceinline__ void rhs3_element(const rhs3_buf<T, P, TX, TY, TZ, KF
 // Stage the tile whose first element is o into B through registers: its coefficient block
 // (zero outside the mesh) and its x and y tables, the backward ones weighted and with
 // -dt*grad folded in.
-template <int NTH = 0, typename T, int P, int TX, int TY, int TZ, bool KF, bool SRC>
-__device__ __forceinline__ void rhs3_stage(rhs3_buf<T, P, TX, TY, TZ, KF, SRC>& B, tile3 o,
+template <int NTH = 0, typename T, int P, int TX, int TY, int TZ, bool KF>
+__device__ __forceinline__ void rhs3_stage(rhs3_buf<T, P, TX, TY, TZ, KF>& B, tile3 o,
                                            const T* __restrict__ up, const dev_tables<T>& X,
                                            const dev_tables<T>& Y, int nz, const rhs_params<T>& prm,
                                            int tid) {
-    using BUF = rhs3_buf<T, P, TX, TY, TZ, KF, SRC>;
+    using BUF = rhs3_buf<T, P, TX, TY, TZ, KF>;
     // NTH: threads of the workgroup (default one per element of the tile)
     constexpr int M = P + 1, NT = NTH ? NTH : TX * TY * TZ, BX = BUF::BX, BY = BUF::BY, NB = BUF::NB;
     static_assert(TX * M * M <= NT && TY * M * M <= NT, "one table entry per thread");
@@ -378,7 +367,6 @@ __device__ __forceinline__ void rhs3_stage(rhs3_buf<T, P, TX, TY, TZ, KF, SRC>& 
         const long g = gx + static_cast<long>(nx) * (gy + static_cast<long>(ny) * gz);
         B.blk[i] = in ? up[g] : T(0);
         if constexpr (KF) B.kb[i] = in ? prm.kfield[g] : T(0);
-        if constexpr (SRC) B.sb[i] = in ? prm.source[g] : T(0);
     }
     const T cx = -prm.dt * prm.gx, cy = -prm.dt * prm.gy;
     if (tid < TX * M * M) {
@@ -423,12 +411,12 @@ __device__ __forceinline__ void lds_fetch(uint32_t* dst, int n, int wave, int la
 // Start copying the tile whose first element is o into B: the coefficient block (indices
 // outside the mesh clamped to the last DOF: those entries are read by no element of the
 // mesh) and the tables as stored (zero-padded per tile; weighted, no -dt*grad).
-template <typename T, int P, int TX, int TY, int TZ, bool KF, bool SRC>
-__device__ __forceinline__ void rhs3_fetch(rhs3_buf<T, P, TX, TY, TZ, KF, SRC>& B, tile3 o,
+template <typename T, int P, int TX, int TY, int TZ, bool KF>
+__device__ __forceinline__ void rhs3_fetch(rhs3_buf<T, P, TX, TY, TZ, KF>& B, tile3 o,
                                            const T* __restrict__ up, const dev_tables<T>& X,
                                            const dev_tables<T>& Y, int nz, const rhs_params<T>& prm,
                                            int wave, int lane) {
-    using BUF = rhs3_buf<T, P, TX, TY, TZ, KF, SRC>;
+    using BUF = rhs3_buf<T, P, TX, TY, TZ, KF>;
     constexpr int M = P + 1, NW = TZ, BX = BUF::BX, BY = BUF::BY, NB = BUF::NB;
     constexpr int DW = sizeof(T) / 4;  // words per value
     const int nx = X.dofs, ny = Y.dofs;
@@ -444,8 +432,6 @@ __device__ __forceinline__ void rhs3_fetch(rhs3_buf<T, P, TX, TY, TZ, KF, SRC>& 
     lds_fetch<NW>(reinterpret_cast<uint32_t*>(B.blk), NB * DW, wave, lane, block_word(up));
     if constexpr (KF)
         lds_fetch<NW>(reinterpret_cast<uint32_t*>(B.kb), NB * DW, wave, lane, block_word(prm.kfield));
-    if constexpr (SRC)
-        lds_fetch<NW>(reinterpret_cast<uint32_t*>(B.sb), NB * DW, wave, lane, block_word(prm.source));
     // the tables: one copy per table, each from a wave-uniform base
     const T* xs[4] = {X.val + static_cast<long>(o.ex0) * M * M, X.der + static_cast<long>(o.ex0) * M * M,
                       X.bval + static_cast<long>(o.ex0) * M * M, X.bder + static_cast<long>(o.ex0) * M * M};
@@ -486,13 +472,13 @@ __device__ __forceinline__ void rhs3_add_block(const double* acc, tile3 o, const
 
 // One workgroup per tile (block b -> tile by XCD-contiguous numbering): tiles of one colour,
 // or (ONE) all ntx2 x nty2 x ntz tiles with the spill array prm.spill.
-template <typename T, int P, int TX, int TY, int TZ, bool KF, bool SRC, int FM, int VAR, bool ONE>
+template <typename T, int P, int TX, int TY, int TZ, bool KF, int FM, int VAR, bool ONE>
 __global__ __launch_bounds__(TX* TY* TZ, (rhs3_waves<T, P, VAR>())) void k_rhs3(
     const T* __restrict__ up, T* __restrict__ rhs, dev_tables<T> X, dev_tables<T> Y,
     dev_tables<T> Z, rhs_params<T> prm, int colour, int ntx2, int nty2) {
     constexpr int NT = TX * TY * TZ, NA = rhs3_acc_size<P, TX, TY, TZ>();
     static_assert(TX * TY == 64, "a wave must cover exactly one z-layer of the tile");
-    __shared__ rhs3_lds<T, P, TX, TY, TZ, KF, SRC, 1> S;
+    __shared__ rhs3_lds<T, P, TX, TY, TZ, KF, 1> S;
     auto& L = S.b[0];
     double* acc = S.acc[0];
 
@@ -509,7 +495,7 @@ __global__ __launch_bounds__(TX* TY* TZ, (rhs3_waves<T, P, VAR>())) void k_rhs3(
     for (int i = tid; i < NA; i += NT) acc[i] = 0.0;
     __syncthreads();
     T R[P + 1][P + 1][P + 1] = {};
-    rhs3_element<T, P, TX, TY, TZ, KF, SRC, FM, VAR>(L, acc, X, Y, Z, prm, lx, ly, lz, o.ex0,
+    rhs3_element<T, P, TX, TY, TZ, KF, FM, VAR>(L, acc, X, Y, Z, prm, lx, ly, lz, o.ex0,
                                                       o.ey0, o.ez0, R);
     __syncthreads();
     const block_sink<T> sink = rhs3_sink<ONE, TX, TY, TZ>(rhs, o, X.elements, Y.elements, Z.elements);
@@ -525,11 +511,11 @@ __global__ __launch_bounds__(TX* TY* TZ, (rhs3_waves<T, P, VAR>())) void k_rhs3(
 // At p = 3 the element's block would not fit the registers: its part for each x point is
 // added to the planes at once.
 template <typename T, int P, int TX, int TY, int TZ>
-__device__ __forceinline__ void kgrad3_element(const rhs3_buf<T, P, TX, TY, TZ, true, false>& L, double* acc,
+__device__ __forceinline__ void kgrad3_element(const rhs3_buf<T, P, TX, TY, TZ, true>& L, double* acc,
                                                const dev_tables<T>& X, const dev_tables<T>& Y,
                                                const dev_tables<T>& Z, const rhs_params<T>& prm, int lx, int ly,
                                                int lz, int ex0, int ey0, int ez0) {
-    using LDS = rhs3_buf<T, P, TX, TY, TZ, true, false>;
+    using LDS = rhs3_buf<T, P, TX, TY, TZ, true>;
     constexpr int M = P + 1, BX = LDS::BX, BY = LDS::BY, PL = LDS::PL;
     constexpr bool FLUSH = P == 3;
     constexpr int RM = FLUSH ? 1 : M;
@@ -684,7 +670,7 @@ __global__ __launch_bounds__(TX* TY* TZ) void k_kgrad3(const T* __restrict__ u, 
                                                      rhs_params<T> prm, int colour, int ntx2, int nty2) {
     constexpr int NT = TX * TY * TZ, NA = rhs3_acc_size<P, TX, TY, TZ>();
     static_assert(TX * TY == 64, "a wave must cover exactly one z-layer of the tile");
-    __shared__ rhs3_lds<T, P, TX, TY, TZ, true, false, 1> S;
+    __shared__ rhs3_lds<T, P, TX, TY, TZ, true, 1> S;
     auto& L = S.b[0];
     double* acc = S.acc[0];
     const int tid = threadIdx.x;
@@ -706,13 +692,13 @@ __global__ __launch_bounds__(TX* TY* TZ) void k_kgrad3(const T* __restrict__ u, 
 // latency is hidden behind that work instead of stalling every workgroup at its start.
 // Each tile has its own DOF planes and both are added to the rhs at the end: no global
 // write precedes the integrations, so their z tables stay in scalar registers.
-template <typename T, int P, int TX, int TY, int TZ, bool KF, bool SRC, int FM>
+template <typename T, int P, int TX, int TY, int TZ, bool KF, int FM>
 __global__ __launch_bounds__(TX* TY* TZ, 2) void k_rhs3_pipe(
     const T* __restrict__ up, T* __restrict__ rhs, dev_tables<T> X, dev_tables<T> Y,
     dev_tables<T> Z, rhs_params<T> prm, int colour, int ntx2, int nty2, int ntiles) {
     constexpr int NT = TX * TY * TZ, NA = rhs3_acc_size<P, TX, TY, TZ>();
     static_assert(TX * TY == 64, "a wave must cover exactly one z-layer of the tile");
-    __shared__ rhs3_lds<T, P, TX, TY, TZ, KF, SRC, 2> S;
+    __shared__ rhs3_lds<T, P, TX, TY, TZ, KF, 2> S;
     auto& B0 = S.b[0];
     auto& B1 = S.b[1];
     double* acc0 = S.acc[0];
@@ -732,13 +718,13 @@ __global__ __launch_bounds__(TX* TY* TZ, 2) void k_rhs3_pipe(
     __syncthreads();
     if (two) rhs3_fetch(B1, o1, up, X, Y, Z.dofs, prm, lz, lane);
     T R0[P + 1][P + 1][P + 1] = {};
-    rhs3_element<T, P, TX, TY, TZ, KF, SRC, FM, 3>(B0, acc0, X, Y, Z, prm, lx, ly, lz, o0.ex0,
+    rhs3_element<T, P, TX, TY, TZ, KF, FM, 3>(B0, acc0, X, Y, Z, prm, lx, ly, lz, o0.ex0,
                                                     o0.ey0, o0.ez0, R0);
     if (two) {
         __builtin_amdgcn_s_waitcnt(kWaitVmem);  // the copies into B1
         __syncthreads();
         T R1[P + 1][P + 1][P + 1] = {};
-        rhs3_element<T, P, TX, TY, TZ, KF, SRC, FM, 3>(B1, acc1, X, Y, Z, prm, lx, ly, lz, o1.ex0,
+        rhs3_element<T, P, TX, TY, TZ, KF, FM, 3>(B1, acc1, X, Y, Z, prm, lx, ly, lz, o1.ex0,
                                                         o1.ey0, o1.ez0, R1);
     }
     __syncthreads();
@@ -755,7 +741,7 @@ __global__ __launch_bounds__(TX* TY* TZ, 2) void k_rhs3_pipe(
 // taller tile re-reads fewer halo planes. Wave w owns the LDS planes of DOF planes 2w ..
 // 2w+P+1; the block add, the colouring and the one-launch tiling are those of the other
 // variants.
-template <typename T, int P, int TX, int TY, int TZ, bool KF, bool SRC, int FM>
+template <typename T, int P, int TX, int TY, int TZ, bool KF, int FM>
 __global__ __launch_bounds__(TX* TY*(TZ / 2), 2) void k_rhs3_zpair(
     const T* __restrict__ up, T* __restrict__ rhs, dev_tables<T> X, dev_tables<T> Y,
     dev_tables<T> Z, rhs_params<T> prm, int colour, int ntx2, int nty2) {
@@ -763,7 +749,7 @@ __global__ __launch_bounds__(TX* TY*(TZ / 2), 2) void k_rhs3_zpair(
     constexpr int PL = BX * BY, NB = PL * (TZ + P), WP = P + 2;  // WP: planes per wave
     static_assert(TX * TY == 64 && TZ % 2 == 0 && TZ >= P, "one wave per pair of layers");
     struct lds_t {
-        rhs3_buf<T, P, TX, TY, TZ, KF, SRC> b;
+        rhs3_buf<T, P, TX, TY, TZ, KF> b;
         double acc[NW * WP * PL];
     };
     __shared__ lds_t S;
@@ -779,7 +765,7 @@ __global__ __launch_bounds__(TX* TY*(TZ / 2), 2) void k_rhs3_zpair(
 
     double* mine = S.acc + w * WP * PL;
     T R[M][M][M] = {};
-    rhs3_element<T, P, TX, TY, TZ, KF, SRC, FM, 4>(S.b, mine, X, Y, Z, prm, lx, ly, 2 * w, o.ex0,
+    rhs3_element<T, P, TX, TY, TZ, KF, FM, 4>(S.b, mine, X, Y, Z, prm, lx, ly, 2 * w, o.ex0,
                                                     o.ey0, o.ez0, R);
 #pragma unroll
     for (int b = 0; b < M; ++b)
@@ -791,7 +777,7 @@ __global__ __launch_bounds__(TX* TY*(TZ / 2), 2) void k_rhs3_zpair(
             for (int c = 0; c < P; ++c) R[a][b][c] = R[a][b][c + 1];
             R[a][b][P] = T(0);
         }
-    rhs3_element<T, P, TX, TY, TZ, KF, SRC, FM, 4>(S.b, mine, X, Y, Z, prm, lx, ly, 2 * w + 1,
+    rhs3_element<T, P, TX, TY, TZ, KF, FM, 4>(S.b, mine, X, Y, Z, prm, lx, ly, 2 * w + 1,
                                                     o.ex0, o.ey0, o.ez0, R);
 #pragma unroll
     for (int c = 0; c < M; ++c)
@@ -893,7 +879,7 @@ __device__ __forceinline__ void rhs2_flush(const T (&R)[P + 1][P + 1], double* _
 // adjoint pair; the element loop of one problem runs in strips (adsg_rhs2_march.hip). The LDS arrays are separate
 // __shared__ objects: gathered into one struct, the compiler read the tables with
 // ds_read2_b64 pairs instead of ds_read_b128 and the p = 3 batch kernel ran 1.5x slower.
-template <typename T, int P, int TX, int TY, bool KF, bool SRC, bool ONE>
+template <typename T, int P, int TX, int TY, bool KF, bool ONE>
 __device__ __forceinline__ void rhs2_tile(const T* __restrict__ up, T* __restrict__ rhs, const dev_tables<T>& X,
                                           const dev_tables<T>& Y, const rhs_params<T>& prm, int colour, int t,
                                           int ntx2) {
@@ -905,7 +891,6 @@ __device__ __forceinline__ void rhs2_tile(const T* __restrict__ up, T* __restric
     static_assert(TX <= 64 && 64 % TX == 0 && TY % WY == 0, "waves must cover whole element rows");
     __shared__ T blk[NB];
     __shared__ T kb[KF ? NB : 1];
-    __shared__ T sb[SRC ? NB : 1];
     __shared__ T fvx[TX * M * M], fdx[TX * M * M], bvx[TX * M * M], bdx[TX * M * M];
     __shared__ T fvy[TY * M * M], fdy[TY * M * M], bvy[TY * M * M], bdy[TY * M * M];
     __shared__ double acc[NW * WR * BX];  // wave w owns DOF rows w*WY .. w*WY+WR-1
@@ -923,7 +908,6 @@ __device__ __forceinline__ void rhs2_tile(const T* __restrict__ up, T* __restric
         const long g = gx + static_cast<long>(nx) * gy;
         blk[i] = in ? up[g] : T(0);
         if constexpr (KF) kb[i] = in ? prm.kfield[g] : T(0);
-        if constexpr (SRC) sb[i] = in ? prm.source[g] : T(0);
     }
     const T cx = -prm.dt * prm.gx, cy = -prm.dt * prm.gy;
     for (int i = tid; i < TX * M * M; i += NT) {
@@ -975,10 +959,10 @@ __device__ __forceinline__ void rhs2_tile(const T* __restrict__ up, T* __restric
                 bx[a] = fvx[(lx * M + qx) * M + a];
                 dx[a] = fdx[(lx * M + qx) * M + a];
             }
-            T A0[M], A1[M], KA[KF ? M : 1], SA[SRC ? M : 1];
+            T A0[M], A1[M], KA[KF ? M : 1];
 #pragma unroll
             for (int b = 0; b < M; ++b) {
-                T s0 = 0, s1 = 0, sk = 0, ss = 0;
+                T s0 = 0, s1 = 0, sk = 0;
 #pragma unroll
                 for (int a = 0; a < M; ++a) {
                     const int li = (lx + a) + BX * (ly + b);
@@ -986,30 +970,26 @@ __device__ __forceinline__ void rhs2_tile(const T* __restrict__ up, T* __restric
                     s0 += bx[a] * cv;
                     s1 += dx[a] * cv;
                     if constexpr (KF) sk += bx[a] * kb[li];
-                    if constexpr (SRC) ss += bx[a] * sb[li];
                 }
                 A0[b] = s0;
                 A1[b] = s1;
                 if constexpr (KF) KA[b] = sk;
-                if constexpr (SRC) SA[b] = ss;
             }
             T K0[M], Kx[M];
 #pragma unroll
             for (int b = 0; b < M; ++b) K0[b] = Kx[b] = T(0);
 #pragma unroll
             for (int qy = 0; qy < M; ++qy) {
-                T u = 0, uy = 0, ux = 0, kv = 0, fv = 0;
+                T u = 0, uy = 0, ux = 0, kv = 0;
 #pragma unroll
                 for (int b = 0; b < M; ++b) {
                     u += By[qy][b] * A0[b];
                     uy += Dy[qy][b] * A0[b];
                     ux += By[qy][b] * A1[b];
                     if constexpr (KF) kv += By[qy][b] * KA[b];
-                    if constexpr (SRC) fv += By[qy][b] * SA[b];
                 }
                 T g0 = mass * u;
                 if (prm.reaction != T(0)) g0 += prm.dt * prm.reaction * u * (T(1) - u);
-                if constexpr (SRC) g0 += prm.dt * fv;
                 T gx = ux, gy = cy * uy;
                 if constexpr (KF) {
                     gx *= kv;
@@ -1178,7 +1158,7 @@ __global__ __launch_bounds__(TX* TY) void k_adjoint2(const T* __restrict__ w, co
                                                      int ntx, int tiles) {
     const int b = static_cast<int>(blockIdx.x);
     if (b < tiles)
-        rhs2_tile<T, P, TX, TY, true, false, true>(w, out_r, X, Y, prm_r, 0, b, ntx);
+        rhs2_tile<T, P, TX, TY, true, true>(w, out_r, X, Y, prm_r, 0, b, ntx);
     else
         kgrad2_tile<T, P, TX, TY, true>(u, w, out_k, X, Y, prm_k, 0, b - tiles, ntx);
 }
@@ -1199,7 +1179,7 @@ __global__ __launch_bounds__(TX* TX) void k_rhs2_batch(const rhs2_item<T>* __res
             hi = mid - 1;
     }
     const rhs2_item<T>& it = items[lo];
-    rhs2_tile<T, P, TX, TX, false, false, false>(it.up, it.rhs, it.X, it.Y, it.prm, colour, b - it.first[colour],
+    rhs2_tile<T, P, TX, TX, false, false>(it.up, it.rhs, it.X, it.Y, it.prm, colour, b - it.first[colour],
                                                  it.ntx2[colour]);
 }
 
@@ -1223,7 +1203,7 @@ struct tile<3, 3> {
     static constexpr int X = 8, Y = 8, Z = 3;
 };
 
-template <typename T, int P, bool KF, bool SRC, int FM, int VAR>
+template <typename T, int P, bool KF, int FM, int VAR>
 hipError_t rhs3_colours(const T* up, T* rhs, const dev_tables<T>* d, const rhs_params<T>& prm,
                         hipStream_t s) {
     using TL = tile<3, P>;
@@ -1242,16 +1222,16 @@ hipError_t rhs3_colours(const T* up, T* rhs, const dev_tables<T>* d, const rhs_p
             const int ntz2 = (d[2].elements + TZ2 - 1) / TZ2, nz22 = (ntz2 - cz + 1) / 2;
             const long tiles2 = static_cast<long>(nx2) * ny2 * nz22;
             if (tiles2 > 0)
-                hipLaunchKernelGGL((k_rhs3_zpair<T, P, TL::X, TL::Y, TZ2, KF, SRC, FM>), dim3(tiles2),
+                hipLaunchKernelGGL((k_rhs3_zpair<T, P, TL::X, TL::Y, TZ2, KF, FM>), dim3(tiles2),
                                    dim3(NT), 0, s, up, rhs, d[0], d[1], d[2], prm, c, nx2, ny2);
         } else if constexpr (VAR == 3) {
-            hipLaunchKernelGGL((k_rhs3_pipe<T, P, TL::X, TL::Y, TL::Z, KF, SRC, FM>),
+            hipLaunchKernelGGL((k_rhs3_pipe<T, P, TL::X, TL::Y, TL::Z, KF, FM>),
                                dim3((tiles + 1) / 2), dim3(NT), 0, s, up, rhs, d[0], d[1], d[2], prm,
                                c, nx2, ny2, static_cast<int>(tiles));
         } else {
             // variant 4 at p = 3 (its register block would spill) runs as variant 2
             constexpr int V = VAR == 4 ? 2 : VAR;
-            hipLaunchKernelGGL((k_rhs3<T, P, TL::X, TL::Y, TL::Z, KF, SRC, FM, V, false>), dim3(tiles),
+            hipLaunchKernelGGL((k_rhs3<T, P, TL::X, TL::Y, TL::Z, KF, FM, V, false>), dim3(tiles),
                                dim3(NT), 0, s, up, rhs, d[0], d[1], d[2], prm, c, nx2, ny2);
         }
         hipError_t e = hipGetLastError();
@@ -1400,7 +1380,7 @@ long spill_layout(const int n[3], const int nt[3], long off[8], int ext[3][2]) {
 }
 
 // One launch over all tiles (variants 0, 1 and 2), then the spill fix-up over the DOFs.
-template <typename T, int P, bool KF, bool SRC, int FM, int VAR>
+template <typename T, int P, bool KF, int FM, int VAR>
 hipError_t rhs3_one(const T* up, T* rhs, const dev_tables<T>* d, const rhs_params<T>& prm, hipStream_t s) {
     using TL = tile<3, P>;
     static_assert(VAR <= 2, "the other variants have no one-launch form here");
@@ -1416,7 +1396,7 @@ hipError_t rhs3_one(const T* up, T* rhs, const dev_tables<T>* d, const rhs_param
     for (int i = 0; i < 3; ++i)
         if (n[i] != d[i].elements + P) return hipErrorInvalidValue;
     spill_layout<P>(n, nt, q.spill_off, q.spill_ext);
-    hipLaunchKernelGGL((k_rhs3<T, P, TL::X, TL::Y, TL::Z, KF, SRC, FM, VAR, true>), dim3(tiles),
+    hipLaunchKernelGGL((k_rhs3<T, P, TL::X, TL::Y, TL::Z, KF, FM, VAR, true>), dim3(tiles),
                        dim3(TL::X * TL::Y * TL::Z), 0, s, up, rhs, d[0], d[1], d[2], q, 0, ntx, nty);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -1501,7 +1481,6 @@ hipError_t kgrad3(const T* u, const T* w, T* out, const dev_tables<T>* d, const 
         if (n[i] != d[i].elements + P) return hipErrorInvalidValue;
     rhs_params<T> q = prm;
     q.kfield = w;  // staged as the k block
-    q.source = nullptr;
     q.store = false;
     q.defer = nullptr;
     if (prm.spill) {
@@ -1562,27 +1541,25 @@ hipError_t kgrad2(const T* u, const T* w, T* out, const dev_tables<T>* d, const 
 template <typename T, int P, int FM, int VAR>
 hipError_t rhs3_forms(const T* up, T* rhs, const dev_tables<T>* d, const rhs_params<T>& prm,
                       hipStream_t s) {
-    const bool kf = prm.kfield != nullptr, src = prm.source != nullptr;
-    if (kf && src) return rhs3_colours<T, P, true, true, FM, VAR>(up, rhs, d, prm, s);
-    if (kf) return rhs3_colours<T, P, true, false, FM, VAR>(up, rhs, d, prm, s);
-    if (src) return rhs3_colours<T, P, false, true, FM, VAR>(up, rhs, d, prm, s);
-    return rhs3_colours<T, P, false, false, FM, VAR>(up, rhs, d, prm, s);
+    const bool kf = prm.kfield != nullptr;
+    if (kf) return rhs3_colours<T, P, true, FM, VAR>(up, rhs, d, prm, s);
+    return rhs3_colours<T, P, false, FM, VAR>(up, rhs, d, prm, s);
 }
 
 template <typename T, int P, int VAR>
 hipError_t rhs3_fields(const T* up, T* rhs, const dev_tables<T>* d, const rhs_params<T>& prm,
                        bool one, hipStream_t s) {
-    // one launch (forms without a k field or a source in the kernel; checked by the caller)
+    // one launch (forms without a k field; checked by the caller)
     if constexpr (VAR <= 2) {
         if (one) {
-            if (prm.reaction != T(0)) return rhs3_one<T, P, false, false, 1, VAR>(up, rhs, d, prm, s);
-            if (prm.mass == T(0)) return rhs3_one<T, P, false, false, 2, VAR>(up, rhs, d, prm, s);
-            return rhs3_one<T, P, false, false, 0, VAR>(up, rhs, d, prm, s);
+            if (prm.reaction != T(0)) return rhs3_one<T, P, false, 1, VAR>(up, rhs, d, prm, s);
+            if (prm.mass == T(0)) return rhs3_one<T, P, false, 2, VAR>(up, rhs, d, prm, s);
+            return rhs3_one<T, P, false, 0, VAR>(up, rhs, d, prm, s);
         }
     }
     if (prm.reaction != T(0)) return rhs3_forms<T, P, 1, VAR>(up, rhs, d, prm, s);
-    if (prm.mass == T(0) && !prm.kfield && !prm.source)
-        return rhs3_colours<T, P, false, false, 2, VAR>(up, rhs, d, prm, s);
+    if (prm.mass == T(0) && !prm.kfield)
+        return rhs3_colours<T, P, false, 2, VAR>(up, rhs, d, prm, s);
     return rhs3_forms<T, P, 0, VAR>(up, rhs, d, prm, s);
 }
 
@@ -1590,15 +1567,15 @@ template <typename T, int P>
 hipError_t rhs_fields(int dim, const T* up, T* rhs, const dev_tables<T>* d,
                       const rhs_params<T>& prm_in, int code, hipStream_t s) {
     rhs_params<T> prm = prm_in;
-    const bool kf = prm.kfield != nullptr, src = prm.source != nullptr;
+    const bool kf = prm.kfield != nullptr;
     // bits 4..7: the shape of variant 5; bit 8: one launch; bit 9: overwrite
     int variant = code & 15;
     if (dim == 3 && variant == 5 && !rhs3_col_supported<T>(P, prm)) variant = P == 3 ? 2 : 1;
     // element columns on the matrix cores where the form allows, else the degree's default
     // per-element variant
-    const bool march = dim == 3 && !src && rhs3_march_fits(sizeof(T), d[0].dofs, d[1].dofs) &&
+    const bool march = dim == 3 && rhs3_march_fits(sizeof(T), d[0].dofs, d[1].dofs) &&
                        (!kf || rhs3_march_kfield<T>(P));
-    const bool one = dim == 3 && (code & kRhsOneLaunch) != 0 && prm.spill && variant != 3 && variant != 5 && !src &&
+    const bool one = dim == 3 && (code & kRhsOneLaunch) != 0 && prm.spill && variant != 3 && variant != 5 &&
                      (!kf || march);
     // 3D in one launch: the marching kernel for variant 4 and for every form with a k field,
     // which the per-element kernels take in colour launches only (70 x 50 x 61, p = 2, FP64: 34 us

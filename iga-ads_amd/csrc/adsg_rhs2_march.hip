@@ -316,7 +316,7 @@ march2_args<T> march2_problem(int p, int rows, const T* up, T* rhs, const dev_ta
 template <typename T>
 hipError_t launch_rhs2_march(int p, const T* up, T* rhs, const dev_tables<T>* d, const rhs_params<T>& prm,
                              hipStream_t s) {
-    if (prm.source || d[0].dofs != d[0].elements + p || d[1].dofs != d[1].elements + p) return hipErrorInvalidValue;
+    if (d[0].dofs != d[0].elements + p || d[1].dofs != d[1].elements + p) return hipErrorInvalidValue;
     const int rows = march2_rows(sizeof(T), {{p, d[0].dofs, d[1].dofs}});
     const march2_args<T> a = march2_problem<T>(p, rows, up, rhs, d[0], d[1], prm);
     const unsigned blocks = static_cast<unsigned>(march2_strips(a));

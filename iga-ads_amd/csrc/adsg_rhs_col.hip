@@ -1,5 +1,5 @@
 // Element-loop RHS, 3D, in columns of elements (variant 5): compute_rhs
-// (validation.hpp:95-119, heat_3d.hpp:49-67) for forms without a k field or a source in the
+// (validation.hpp:95-119, heat_3d.hpp:49-67) for forms without a k field in the
 // kernel, with the x-y contractions on the matrix cores (MFMA 16x16x4, FP64 or FP32).
 //
 // One wave integrates one column of elements (ex, ey, ez = z0 .. z1-1), walking it in chunks
@@ -409,7 +409,7 @@ hipError_t col_forms(const T* up, T* rhs, const dev_tables<T>* d, const rhs_para
 
 template <typename T>
 bool rhs3_col_supported(int p, const rhs_params<T>& prm) {
-    return (p == 2 || p == 3) && !prm.kfield && !prm.source;
+    return (p == 2 || p == 3) && !prm.kfield;
 }
 
 template <typename T>

@@ -1,7 +1,7 @@
 // Element-loop RHS for any quadrature order, repeated interior knots and a degree per
 // direction (dim_config of simulation/config.hpp:11-56: quad_order, repeated_nodes, p per
 // direction): the loop of validation.hpp:100-118 as written there, one lane per element.
-// At every Gauss point the state (and k, f) and its gradient are evaluated from the
+// At every Gauss point the state (and k) and its gradient are evaluated from the
 // element's (p_x+1)(p_y+1)(p_z+1) coefficients, the integrand is formed and its products
 // with the element's test functions are accumulated; the element's block is then added to
 // the rhs at its first DOFs (bspline.cpp:162-172 first_nonzero_dofs, which repeated knots
@@ -31,9 +31,9 @@ __global__ __launch_bounds__(256) void k_rhs_gen(const T* __restrict__ up, T* __
     if (ex >= X.elements || ey >= Y.elements || (DIM == 3 && ez >= Z.elements)) return;
     const long nx = X.dofs, ny = Y.dofs;
     const int fx = X.first[ex], fy = Y.first[ey], fz = DIM == 3 ? Z.first[ez] : 0;
-    const bool KF = prm.kfield != nullptr, SRC = prm.source != nullptr;
+    const bool KF = prm.kfield != nullptr;
 
-    T U[MZ][MY][MX], Kc[MZ][MY][MX], Fc[MZ][MY][MX];
+    T U[MZ][MY][MX], Kc[MZ][MY][MX];
     double R[MZ][MY][MX];
 #pragma unroll
     for (int c = 0; c < MZ; ++c)
@@ -44,7 +44,6 @@ __global__ __launch_bounds__(256) void k_rhs_gen(const T* __restrict__ up, T* __
                 const long g = (fx + a) + nx * ((fy + b) + ny * static_cast<long>(fz + c));
                 U[c][b][a] = up[g];
                 Kc[c][b][a] = KF ? prm.kfield[g] : T(0);
-                Fc[c][b][a] = SRC ? prm.source[g] : T(0);
                 R[c][b][a] = 0.0;
             }
     const int qz_end = DIM == 3 ? Z.nq : 1;
@@ -79,7 +78,7 @@ __global__ __launch_bounds__(256) void k_rhs_gen(const T* __restrict__ up, T* __
                 }
                 const T w = X.wj[static_cast<long>(ex) * X.nq + qx] * wyz;
                 // eval_fun (simulation_3d.hpp:120-128): value and gradient at the point
-                T u = 0, ux = 0, uy = 0, uz = 0, k = 0, f = 0;
+                T u = 0, ux = 0, uy = 0, uz = 0, k = 0;
 #pragma unroll
                 for (int c = 0; c < MZ; ++c)
 #pragma unroll
@@ -92,11 +91,10 @@ __global__ __launch_bounds__(256) void k_rhs_gen(const T* __restrict__ up, T* __
                             uy += bz[c] * dy[b] * bx[a] * U[c][b][a];
                             if constexpr (DIM == 3) uz += dz[c] * by[b] * bx[a] * U[c][b][a];
                             k += v * Kc[c][b][a];
-                            f += v * Fc[c][b][a];
                         }
                 if (!KF) k = T(1);
                 // the integrand of compute_rhs against v = B_a B_b B_c and its gradient
-                const T g0 = w * (prm.mass * u + prm.dt * prm.reaction * u * (T(1) - u) + (SRC ? prm.dt * f : T(0)));
+                const T g0 = w * (prm.mass * u + prm.dt * prm.reaction * u * (T(1) - u));
                 const T gk = -w * prm.dt * k;
                 const T gx = gk * prm.gx * ux, gy = gk * prm.gy * uy, gz = gk * prm.gz * uz;
 #pragma unroll

@@ -515,7 +515,7 @@ hipError_t march_forms(const T* up, T* rhs, const dev_tables<T>* d, const rhs_pa
 template <typename T>
 hipError_t launch_rhs3_march(int p, const T* u_prev, T* rhs, const dev_tables<T>* dirs, const rhs_params<T>& prm,
                              const int tile[3], const int nt[3], hipStream_t s) {
-    if (prm.source || !prm.spill) return hipErrorInvalidValue;
+    if (!prm.spill) return hipErrorInvalidValue;
     switch (p) {
         case 1:
             return march_forms<T, 1>(u_prev, rhs, dirs, prm, tile, nt, s);
