@@ -1267,8 +1267,7 @@ int adsg_prepare_matrices(adsg_sim* h) {
             }
             s.seg = adsg::line_segments{};
             // up to 16 segment waves (1024 lanes) of 16 or 32 rows; x lines are staged through
-            // LDS where that fits (150 KB: FP64 14 waves of 16 rows or 8 of 32, FP32 16 or 13)
-            // and read lane by lane otherwise
+            // LDS, 16 lines per workgroup
             if (adsg::segment_lines(s.lf, s.seg, 16, 16)) {
                 if (h->precision == ADSG_FP32) {
                     if ((rc = upload<float>(h, &s.pack, s.seg.pack))) return rc;
