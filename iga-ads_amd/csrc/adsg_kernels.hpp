@@ -196,9 +196,10 @@ hipError_t launch_rhs3_col(int p, const T* u_prev, T* rhs, const dev_tables<T>* 
 // Variant 4 in one launch (adsg_rhs_march.hip): its tiles (elements per tile and tile counts
 // per direction) for degree p, values of `bytes` bytes, with or without a k field; and its
 // launch on them (prm: the spill layout of these tiles set).
-// Forms with a k field: not FP32 at p = 3, where the sums along z in FP32 were 10 to 22 % further
-// from FP64 than the per-element kernels' sums across elements in FP64 (10 heat steps, 64^3 and
-// 128 x 100 x 90); everywhere else its FP32 error is no larger than theirs.
+// Forms with a k field: not FP32 at p = 3, which was only tried with sums along z in FP32 (10 to
+// 22 % further from FP64 than the per-element kernels). With the sums of different elements in FP64
+// its FP32 rhs is 0.15 to 1.02 times as far from FP64 as theirs (heat, reaction, k field and source
+// forms, 9 x 12 x 10 to 110 x 100 x 90, 16 smooth states with 1e-3 of noise).
 template <typename T>
 constexpr bool rhs3_march_kfield(int p) {
     return sizeof(T) == sizeof(double) || p < 3;

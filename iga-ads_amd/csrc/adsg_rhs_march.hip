@@ -30,14 +30,16 @@ namespace {
 // per lane and plane at p = 3 without a mass term, 36 per Gauss point column; the per-element
 // kernel spends 4768 multiply-adds per element, this one about 2400.
 // Bound: FP64 issue (1.85 ns per wave instruction and SIMD, dependent or not). The element
-// pass of 192^3, p = 3, FP64 without a mass term went from 2197 to 960 us (FP32 from 1197 us
-// on the matrix cores to 625), 128^3, p = 2 from 165 to 141 us (FP32 98 to 92), with a k field
-// (70 x 50 x 61, p = 2) from 154 us in colour launches to 46. Measured on the way: lanes over
+// pass of 192^3, p = 3, FP64 without a mass term went from 2197 to 893 us (FP32 from 1197 us
+// on the matrix cores to 689), 128^3, p = 2 from 165 to 136 us (FP32 98 to 103, with shorter
+// sweeps after it than the kernels that were replaced had), with a k field (70 x 50 x 61, p = 2)
+// from 154 us in colour launches to 34. Measured on the way: lanes over
 // element pairs of y Gauss points at twice the waves (more instructions, 1.5x slower); the z
 // tables as DPP broadcast operands instead of scalar registers (more registers: spills); the
 // x contraction one plane ahead and the block write spread over the planes (registers again:
-// 3 to 20 % slower). What is left is the register file: 2 waves per SIMD at p = 3 FP64, 3
-// elsewhere, leave a third of the issue slots to LDS and scalar-load latency and barriers.
+// 3 to 20 % slower). What is left is the register file: at p = 3 FP64 the 256 registers of 2
+// waves per SIMD hold all but 39 to 72 of the values (scratch), and 2 or 3 waves hide little of
+// the LDS and scalar-load latency.
 // ------------------------------------------------------------------------------------
 template <int P>
 struct march {
@@ -54,10 +56,10 @@ struct march {
 // slower: the SIMD with two of them sets the pace between the barriers; eight 1.2x)
 constexpr int kMarchRows = 4;
 // waves per SIMD the register allocation must allow: the window of M planes and the sums of M
-// planes are 6 M^2 values per lane (7 M^2 with a k field)
-template <typename T, int P, bool KF>
-constexpr int march_waves() {
-    return sizeof(T) == sizeof(float) ? 3 : P == 3 ? (KF ? 1 : 2) : P == 2 && KF ? 2 : 3;
+// planes are 6 M^2 values per lane (7 M^2 with a k field), the sums FP64 in both precisions (FP32
+// at p = 3 in 3 waves: 214 registers spilled)
+constexpr int march_waves(int bytes, int p, bool kfield) {
+    return p == 3 ? (bytes == 8 && kfield ? 1 : 2) : bytes == 8 && p == 2 && kfield ? 2 : 3;
 }
 
 template <typename T, int P, bool KF>
@@ -97,7 +99,7 @@ __device__ __forceinline__ const T* at(const T* base, unsigned bytes) {
 
 // FM: 0 the heat form (mass term), 1 with the reaction term, 2 no mass term, KF: k field
 template <typename T, int P, bool KF, int FM>
-__global__ __launch_bounds__((64 * kMarchRows), (march_waves<T, P, KF>())) void k_rhs3_march(march_args<T> A) {
+__global__ __launch_bounds__((64 * kMarchRows), march_waves(sizeof(T), P, KF)) void k_rhs3_march(march_args<T> A) {
     using S = march<P>;
     using L = march_lds<T, P, KF>;
     constexpr int M = P + 1, TX = S::TX, TY = kMarchRows, BX = S::BX, NL = S::NL, SX = S::SX, RP = S::RP;
@@ -194,19 +196,15 @@ __global__ __launch_bounds__((64 * kMarchRows), (march_waves<T, P, KF>())) void 
 #pragma unroll
         for (int j = 0; j < NL; ++j) asm volatile("" : "+v"(i_sr[j]), "+v"(i_pw[j]));
     };
-    // FP32 without a mass term: gradients only, so a constant may be taken from the row's
-    // coefficients (exactly, or to the rounding of the difference): the contractions then round
-    // relative to the variation of u along the march instead of to u
-    constexpr bool REL = sizeof(T) == sizeof(float) && !MS;
-    T uref = T(0);
-    if constexpr (REL) {
-        uref = A.up[min(ex0 + TX / 2, nx - 1) + static_cast<long>(nx) * min(ey0 + wv, ny - 1) + (ez0 + npl / 2) * pstride];
-        if (!(uref - uref == T(0))) uref = T(0);  // not finite: it stays where it is
-    }
+    // FP32: the contractions take differences from the element's first coefficient (its first row,
+    // its first plane), which the derivatives are made of: their rounding errors scale with the
+    // variation of u over the element (the basis functions sum to 1, their derivatives to 0).
+    // The sums of different elements are FP64 in both precisions.
+    constexpr bool REL = sizeof(T) == sizeof(float);
     auto stage = [&]() {
 #pragma unroll
         for (int j = 0; j < NL; ++j) {
-            ub[j * 64 + i_lane] = REL ? pre[j] - uref : pre[j];
+            ub[j * 64 + i_lane] = pre[j];
             if constexpr (KF) ub[(NL + j) * 64 + i_lane] = prek[j];
         }
     };
@@ -219,11 +217,15 @@ __global__ __launch_bounds__((64 * kMarchRows), (march_waves<T, P, KF>())) void 
     };
 
     T w00[M][M], w01[M][M], w10[M][M], wk[KF ? M : 1][KF ? M : 1];  // [plane mod M][y Gauss point]
-    T h0[M][M], hx[M][M], hy[M][M];
+    T w0[REL ? M : 1];  // [plane mod M]: the coefficient that w00 is relative to
+    double h0[M][M], hx[M][M], hy[M][M];
 #pragma unroll
     for (int s = 0; s < M; ++s)
 #pragma unroll
-        for (int y = 0; y < M; ++y) w00[s][y] = w01[s][y] = w10[s][y] = h0[s][y] = hx[s][y] = hy[s][y] = T(0);
+        for (int y = 0; y < M; ++y) {
+            w00[s][y] = w01[s][y] = w10[s][y] = T(0);
+            h0[s][y] = hx[s][y] = hy[s][y] = 0.0;
+        }
     const T* ytab = A.tab[1] + static_cast<long>(ey0 + (act ? wv : 0)) * TAB;
 
     // the block write of the M planes from e0 on, from part buffer par
@@ -276,33 +278,43 @@ __global__ __launch_bounds__((64 * kMarchRows), (march_waves<T, P, KF>())) void 
             wave_lds_sync();
             T A0[M], A1[M], AK[KF ? M : 1];
             {  // U: the rows of plane k along x
-                T fv[M], fd[M];
+                T fv[M], fd[M], r[M];
                 load_tab(0, fv, fd);
 #pragma unroll
                 for (int b = 0; b < M; ++b) {
                     T a0 = 0, a1 = 0, ak = 0;
+                    r[b] = ub[i_el + b * BX];
 #pragma unroll
                     for (int a = 0; a < M; ++a) {
-                        const T v = ub[i_el + b * BX + a];
-                        a0 += fv[a] * v;
-                        a1 += fd[a] * v;
+                        const T v = a == 0 ? r[b] : ub[i_el + b * BX + a];
+                        if (!REL || a > 0) {
+                            a0 += fv[a] * (REL ? v - r[b] : v);
+                            a1 += fd[a] * (REL ? v - r[b] : v);
+                        }
                         if constexpr (KF) ak += fv[a] * ub[i_el + NL * 64 + b * BX + a];
                     }
                     A0[b] = a0;
                     A1[b] = a1;
                     if constexpr (KF) AK[b] = ak;
                 }
+                if constexpr (REL) {
+                    w0[kk] = r[0];
+#pragma unroll
+                    for (int b = 1; b < M; ++b) A0[b] = (A0[b] - A0[0]) + (r[b] - r[0]);
+                }
             }
             const T* yt = ytab;
             asm volatile("" : "+s"(yt));  // the y tables are re-read per plane, not kept
 #pragma unroll
             for (int y = 0; y < M; ++y) {  // Y
-                T s00 = 0, s01 = 0, s10 = 0, sk = 0;
+                T s00 = REL ? A0[0] : T(0), s01 = 0, s10 = 0, sk = 0;
 #pragma unroll
                 for (int b = 0; b < M; ++b) {
                     const T bv = uniform_load(yt + y * 4 * M + b), bd = uniform_load(yt + (y * 4 + 1) * M + b);
-                    s00 += bv * A0[b];
-                    s01 += bd * A0[b];
+                    if (!REL || b > 0) {
+                        s00 += bv * A0[b];
+                        s01 += bd * A0[b];
+                    }
                     s10 += bv * A1[b];
                     if constexpr (KF) sk += bv * AK[b];
                 }
@@ -316,11 +328,13 @@ __global__ __launch_bounds__((64 * kMarchRows), (march_waves<T, P, KF>())) void 
             auto points = [&](auto zstage) {
                 const T* zt = A.tab[2] + static_cast<long>(ez0 + e) * TAB;
                 T tv[M], td[M];
+                // (FP32: the z points of a y point together, their sums then added in FP64)
+                T dz[M], l0[M], lx[M], ly[M];
 #pragma unroll
                 for (int p = 0; p < M * M; ++p) {
-                    const int z = p / M, y = p % M, b = p / M;
+                    const int z = REL ? p % M : p / M, y = REL ? p / M : p % M, b = p / M;
                     T v[M], vx[M];
-                    if (y == 0) {
+                    if (p % M == 0) {
                         if (b == 0) load_tab(2, tv, td);
 #pragma unroll
                         for (int r = 0; r < M; ++r) {
@@ -337,12 +351,23 @@ __global__ __launch_bounds__((64 * kMarchRows), (march_waves<T, P, KF>())) void 
                             zbv[c] = uniform_load(zt + (z * 4 + 2) * M + c);
                             zbd[c] = uniform_load(zt + (z * 4 + 3) * M + c);
                         }
-                        T u = 0, ux = 0, uy = 0, uz = 0, kv = 0;
+                        if (REL && z == 0) {  // dz[c]: plane c relative to the first one
+                            const int s0 = (kk + 1) % M;
+                            dz[0] = w00[s0][y] + w0[REL ? s0 : 0];
+#pragma unroll
+                            for (int c = 1; c < M; ++c) {
+                                const int s = (kk + 1 + c) % M;
+                                dz[c] = (w00[s][y] - w00[s0][y]) + (w0[REL ? s : 0] - w0[REL ? s0 : 0]);
+                            }
+                        }
+                        T u = REL ? dz[0] : T(0), ux = 0, uy = 0, uz = 0, kv = 0;
 #pragma unroll
                         for (int c = 0; c < M; ++c) {
                             const int s = (kk + 1 + c) % M;
-                            if constexpr (MS) u += zv[c] * w00[s][y];
-                            uz += zd[c] * w00[s][y];
+                            if (!REL || c > 0) {
+                                if constexpr (MS) u += zv[c] * (REL ? dz[c] : w00[s][y]);
+                                uz += zd[c] * (REL ? dz[c] : w00[s][y]);
+                            }
                             uy += zv[c] * w01[s][y];
                             ux += zv[c] * w10[s][y];
                             if constexpr (KF) kv += zv[c] * wk[KF ? s : 0][KF ? y : 0];
@@ -360,6 +385,18 @@ __global__ __launch_bounds__((64 * kMarchRows), (march_waves<T, P, KF>())) void 
 #pragma unroll
                         for (int c = 0; c < M; ++c) {
                             const int s = (kk + 1 + c) % M;
+                            if constexpr (REL) {
+                                l0[c] = z == 0 ? zbd[c] * gz : l0[c] + zbd[c] * gz;
+                                lx[c] = z == 0 ? zbv[c] * gx : lx[c] + zbv[c] * gx;
+                                ly[c] = z == 0 ? zbv[c] * gy : ly[c] + zbv[c] * gy;
+                                if constexpr (MS) l0[c] += zbv[c] * g0;
+                                if (z == P) {
+                                    h0[s][y] = c == P ? l0[c] : h0[s][y] + l0[c];
+                                    hx[s][y] = c == P ? lx[c] : hx[s][y] + lx[c];
+                                    hy[s][y] = c == P ? ly[c] : hy[s][y] + ly[c];
+                                }
+                                continue;
+                            }
                             if (c == P && z == 0) {  // the element's last plane: its first contribution
                                 h0[s][y] = zbd[c] * gz;
                                 hx[s][y] = zbv[c] * gx;
@@ -372,7 +409,7 @@ __global__ __launch_bounds__((64 * kMarchRows), (march_waves<T, P, KF>())) void 
                             if constexpr (MS) h0[s][y] += zbv[c] * g0;
                         }
                     }
-                    if (y == 0) {
+                    if (p % M == 0) {
                         T s = 0;
 #pragma unroll
                         for (int r = 0; r < M; ++r) {
@@ -405,9 +442,9 @@ __global__ __launch_bounds__((64 * kMarchRows), (march_waves<T, P, KF>())) void 
 #pragma unroll
                     for (int y = 0; y < M; ++y) {
                         const T bv = uniform_load(yt + (y * 4 + 2) * M + b), bd = uniform_load(yt + (y * 4 + 3) * M + b);
-                        K0 += bv * h0[s][y];
-                        Ky += bd * hy[s][y];
-                        Kx += bv * hx[s][y];
+                        K0 += bv * static_cast<T>(h0[s][y]);
+                        Ky += bd * static_cast<T>(hy[s][y]);
+                        Kx += bv * static_cast<T>(hx[s][y]);
                     }
                     kb[b * 64 + i_lane] = MS ? K0 + A.cy * Ky : A.cz * K0 + A.cy * Ky;
                     kb[(M + b) * 64 + i_lane] = Kx;
@@ -445,7 +482,7 @@ void march_tiles(int waves, const int el[3], int tile[3]) {
 }  // namespace
 
 void rhs3_march_tiles(int p, int bytes, bool kfield, const int elements[3], int tile[3], int nt[3]) {
-    const int waves = bytes == 4 ? 3 : p == 3 ? (kfield ? 1 : 2) : p == 2 && kfield ? 2 : 3;
+    const int waves = march_waves(bytes, p, kfield);
     if (p == 1) march_tiles<1>(waves, elements, tile);
     if (p == 2) march_tiles<2>(waves, elements, tile);
     if (p == 3) march_tiles<3>(waves, elements, tile);
