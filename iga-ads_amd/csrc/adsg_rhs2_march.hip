@@ -20,8 +20,9 @@ namespace {
 //  X  its M = P + 1 coefficients of the row contracted along x at its M Gauss points (value,
 //     derivative), kept in registers for the M rows that an element row reads,
 //  Y  for the element row that begins at this DOF row: along y to the M^2 Gauss points, the
-//     integrand, and its y-transposed sums, kept in registers for the M rows it touches,
-//  S  the row is complete: x transposed, the M contributions to neighbouring columns summed
+//     integrand, and its y-transposed sums (FP32: transposed in x too), kept in FP64 registers
+//     for the M rows it touches,
+//  S  the row is complete: x transposed (FP64), the M contributions to neighbouring columns summed
 //     by shifting them across the lanes, stored.
 // The x contractions run once per DOF row instead of once per element, and every DOF is
 // written once by one lane in a fixed order: no colours, no spill entries, no LDS. What it
@@ -29,14 +30,13 @@ namespace {
 // Bound: instruction issue, and in small problems the serial P + 1 element rows of a strip.
 // Whole steps, us, element kernel in 16 x 16 tiles (four colour launches in batches, one launch
 // and a spill fix-up for one problem) and here: 256 problems of 32 to 256 elements FP32 289 ->
-// 183 (of them the element kernels 186 -> 95), 24 of 32 to 90 110 -> 35, 96 of 32 to 200 FP64
+// 191 (of them the element kernels 186 -> 96), 24 of 32 to 90 110 -> 36, 96 of 32 to 200 FP64
 // 155 -> 103 (sweeps and all). One problem, FP64, element kernel and fix-up: 128 x 128 p = 2
 // with a k field 8.3 -> 5.6, 480 x 351 p = 3 25 -> 17.
 // ------------------------------------------------------------------------------------
 
 // lane l: the value of lane l - 1, 0 in lane 0 (DPP wave_shr:1)
 __device__ __forceinline__ int lane_below(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, false); }
-__device__ __forceinline__ float lane_below(float v) { return __int_as_float(lane_below(__float_as_int(v))); }
 __device__ __forceinline__ double lane_below(double v) {
     return __hiloint2double(lane_below(__double2hiint(v)), lane_below(__double2loint(v)));
 }
@@ -101,11 +101,24 @@ __device__ __forceinline__ void march2_strip(const march2_args<T>& A, int t) {
             if constexpr (KF) k[j][q] = sk;
         }
     };
-    T V[M][M], D[M][M];  // sums of row r + j: against values and x derivatives
+    // The sums of row r + j. The sums of different elements are FP64 in both precisions. FP64:
+    // against values (V) and x derivatives (D) at the lane's Gauss points, x transposed once per
+    // row. FP32: an element's contributions are complete in FP32 before they are added, R[j][i] to
+    // its column i: sums across element rows first and x transposed after them in FP32 were 10 to
+    // 20 % further from FP64 on rough states (and tables with the weights folded in up to 30 % at
+    // p = 1: their rounding is the same in every element).
+    constexpr bool F32 = sizeof(T) == sizeof(float);
+    constexpr int MV = F32 ? 1 : M, MR = F32 ? M : 1;
+    double V[MV][MV], D[MV][MV], R[MR][MR];
+    const T cx = A.cx;
 #pragma unroll
-    for (int j = 0; j < M; ++j)
+    for (int j = 0; j < MV; ++j)
 #pragma unroll
-        for (int q = 0; q < M; ++q) V[j][q] = D[j][q] = T(0);
+        for (int q = 0; q < MV; ++q) V[j][q] = D[j][q] = 0.0;
+#pragma unroll
+    for (int j = 0; j < MR; ++j)
+#pragma unroll
+        for (int i = 0; i < MR; ++i) R[j][i] = 0.0;
     fetch(b0);
 #pragma unroll
     for (int j = 0; j < P; ++j) {
@@ -131,18 +144,20 @@ __device__ __forceinline__ void march2_strip(const march2_args<T>& A, int t) {
 #pragma unroll
                     for (int c = 1; c < M; ++c) da[c][q] = (a[c][q] - a[0][q]) + (u0[c] - u0[0]);
                 }
+                T lv[M], ld[M], sum[MR][MR];  // FP32: the y points of an x point, its sums; the element's
 #pragma unroll
-                for (int y = 0; y < M; ++y) {
-                    T v[M], g[M];
+                for (int o = 0; o < M; ++o) {
 #pragma unroll
-                    for (int c = 0; c < M; ++c) {
-                        v[c] = (uniform_load(yv + y * M + c));
-                        g[c] = (uniform_load(yd + y * M + c));
-                    }
-                    const T w = (uniform_load(yw + y)), wc = w * A.cy;
-                    const T wm = VAL == 2 ? w * (A.mass + A.rdt) : w * A.mass, wr = w * A.rdt;
+                    for (int i = 0; i < M; ++i) {
+                        const int y = F32 ? i : o, q = F32 ? o : i;
+                        T v[M], g[M];
 #pragma unroll
-                    for (int q = 0; q < M; ++q) {
+                        for (int c = 0; c < M; ++c) {
+                            v[c] = (uniform_load(yv + y * M + c));
+                            g[c] = (uniform_load(yd + y * M + c));
+                        }
+                        const T w = (uniform_load(yw + y)), wc = w * A.cy;
+                        const T wm = VAL == 2 ? w * (A.mass + A.rdt) : w * A.mass, wr = w * A.rdt;
                         T u = da[0][q], ux = 0, uy = 0, kv = 0;
 #pragma unroll
                         for (int c = 0; c < M; ++c) {
@@ -161,9 +176,25 @@ __device__ __forceinline__ void march2_strip(const march2_args<T>& A, int t) {
                         u *= VAL == 2 ? mad(-wr, u, wm) : wm;  // w (mass u + dt reaction u (1 - u))
 #pragma unroll
                         for (int c = 0; c < M; ++c) {
-                            V[c][q] = mad(g[c], gy, V[c][q]);
-                            if constexpr (VAL > 0) V[c][q] = mad(v[c], u, V[c][q]);
-                            D[c][q] = mad(v[c], gx, D[c][q]);
+                            if constexpr (F32) {
+                                lv[c] = y == 0 ? g[c] * gy : mad(g[c], gy, lv[c]);
+                                if constexpr (VAL > 0) lv[c] = mad(v[c], u, lv[c]);
+                                ld[c] = y == 0 ? v[c] * gx : mad(v[c], gx, ld[c]);
+                                if (y == P) {
+                                    lv[c] *= wx[q];
+                                    ld[c] *= cx * wx[q];
+#pragma unroll
+                                    for (int x = 0; x < M; ++x) {
+                                        sum[c][x] = q == 0 ? bv[q][x] * lv[c] : mad(bv[q][x], lv[c], sum[c][x]);
+                                        sum[c][x] = mad(bd[q][x], ld[c], sum[c][x]);
+                                        if (q == P) R[c][x] += sum[c][x];
+                                    }
+                                }
+                            } else {
+                                V[c][q] = mad(g[c], gy, V[c][q]);
+                                if constexpr (VAL > 0) V[c][q] = mad(v[c], u, V[c][q]);
+                                D[c][q] = mad(v[c], gx, D[c][q]);
+                            }
                         }
                     }
                 }
@@ -175,19 +206,21 @@ __device__ __forceinline__ void march2_strip(const march2_args<T>& A, int t) {
             else
                 element(std::integral_constant<int, 0>{});
         }
-        // row r is complete (p = 3: its columns' contributions summed in FP64 in both precisions,
-        // for cancelling fluxes on coarse meshes)
-        using S = std::conditional_t<P == 3, double, T>;
-        S s = 0;
+        // row r is complete
+        double s = 0;
 #pragma unroll
         for (int i = P; i >= 0; --i) {
-            T c = 0;
+            double c = 0;
+            if constexpr (F32) {
+                c = R[0][i];
+            } else {
 #pragma unroll
-            for (int q = 0; q < M; ++q) {
-                c = mad(bv[q][i], wx[q] * V[0][q], c);
-                c = mad(bd[q][i], (A.cx * wx[q]) * D[0][q], c);
+                for (int q = 0; q < M; ++q) {
+                    c = mad(bv[q][i], wx[q] * V[0][q], c);
+                    c = mad(bd[q][i], (cx * wx[q]) * D[0][q], c);
+                }
             }
-            s = (i < P ? lane_below(s) : S(0)) + static_cast<S>(in ? c : T(0));
+            s = (i < P ? lane_below(s) : 0.0) + (in ? c : 0.0);
         }
         if (r >= r0 && own) {
             const long o = static_cast<long>(A.nx) * r;
@@ -201,12 +234,21 @@ __device__ __forceinline__ void march2_strip(const march2_args<T>& A, int t) {
                 a[j][q] = a[j + 1][q];
                 d[j][q] = d[j + 1][q];
                 if constexpr (KF) k[j][q] = k[j + 1][q];
-                V[j][q] = V[j + 1][q];
-                D[j][q] = D[j + 1][q];
+                if constexpr (F32) {
+                    R[j][q] = R[j + 1][q];
+                } else {
+                    V[j][q] = V[j + 1][q];
+                    D[j][q] = D[j + 1][q];
+                }
             }
         }
 #pragma unroll
-        for (int q = 0; q < M; ++q) V[P][q] = D[P][q] = T(0);
+        for (int q = 0; q < M; ++q) {
+            if constexpr (F32)
+                R[P][q] = 0.0;
+            else
+                V[P][q] = D[P][q] = 0.0;
+        }
     }
 }
 
