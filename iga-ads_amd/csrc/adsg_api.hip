@@ -1926,10 +1926,12 @@ int adsg_autotune(adsg_sim* h, const adsg_rhs_form* form, const int* slots, int 
                 hit = true;
             }
         }
-        if (hit && (c[2] == 0 || ensure_spill(h) == ADSG_OK)) {
-            h->rhs_variant = c[0];
-            h->rhs_col_shape = c[1];
-            h->rhs_tiling = c[2];
+        if (hit && (h->dim == 2 || c[2] == 0 || ensure_spill(h) == ADSG_OK)) {
+            if (h->dim == 3) {
+                h->rhs_variant = c[0];
+                h->rhs_col_shape = c[1];
+                h->rhs_tiling = c[2];
+            }
             h->sweep_variant = c[3];
             drop_graphs(h);
             return ADSG_OK;
@@ -1958,17 +1960,21 @@ int adsg_autotune(adsg_sim* h, const adsg_rhs_form* form, const int* slots, int 
     double best_ms = 1e30, best_sweep_ms = 1e30;
     int rc = ADSG_OK;
     // candidates {variant, shape of variant 5, tiling}: variants 0..4 in colour launches, the
-    // column variant (5) in each of its shapes, and (3D) variants 0, 1, 2, 4 in one launch
+    // column variant (5) in each of its shapes, and variants 0, 1, 2, 4 in one launch. In 2D the
+    // element loop is the same kernel with each of them, and the tiling is that of the k-field
+    // gradients, which a step does not time: only the sweep variants are timed there.
     std::vector<std::array<int, 3>> cand;
-    for (int v = 0; v <= 4; ++v) cand.push_back({v, 0, 0});
-    for (int c = 0; c <= 3; ++c) cand.push_back({5, c, 0});
-    if (!h->general && ensure_spill(h) == ADSG_OK && h->spill)
-        for (int v : (h->dim == 3 ? std::vector<int>{0, 1, 2, 4} : std::vector<int>{0})) cand.push_back({v, 0, 1});
+    for (int v = 0; v <= (h->dim == 3 ? 4 : 2); ++v) cand.push_back({v, 0, 0});
+    for (int c = 0; c <= 3 && h->dim == 3; ++c) cand.push_back({5, c, 0});
+    if (h->dim == 3 && !h->general && ensure_spill(h) == ADSG_OK && h->spill)
+        for (int v : {0, 1, 2, 4}) cand.push_back({v, 0, 1});
     for (size_t k = 0; k < cand.size() && rc == ADSG_OK; ++k) {
         const int v = cand[k][0];
-        h->rhs_variant = v;
-        h->rhs_col_shape = cand[k][1];
-        h->rhs_tiling = cand[k][2];
+        if (h->dim == 3) {
+            h->rhs_variant = v;
+            h->rhs_col_shape = cand[k][1];
+            h->rhs_tiling = cand[k][2];
+        }
         // the sweep variants 0, 1, 2 timed with the element variants of the same number in
         // colour launches
         const bool sweep_run = v <= 2 && cand[k][2] == 0;
@@ -1977,7 +1983,7 @@ int adsg_autotune(adsg_sim* h, const adsg_rhs_form* form, const int* slots, int 
         rc = adsg_time_phases(h, 1, form, slots, flags, ms);  // warm-up (code load, caches)
         // 8 timed steps: variants 1 and 3 are a few per cent apart at full-GPU sizes
         if (!rc) rc = adsg_time_phases(h, 8, form, slots, flags, ms);
-        if (!rc && ms[0] < best_ms) {
+        if (!rc && h->dim == 3 && ms[0] < best_ms) {
             best_ms = ms[0];
             best = v;
             best_shape = h->rhs_col_shape;

@@ -323,7 +323,8 @@ int adsg_time_phases(adsg_sim* h, int nsteps, const adsg_rhs_form* form, const i
  * by lane).
  * adsg_autotune times every variant on the handle's current state with the given form
  * (explicit steps, or delta steps with slots) and keeps the fastest of each; the state
- * vectors are restored afterwards. */
+ * vectors are restored afterwards. In 2D, where every element variant and tiling runs the same
+ * element kernel, it times the line sweeps and leaves the element settings as they are. */
 #define ADSG_TUNE_RHS_VARIANT 0
 #define ADSG_TUNE_SWEEP_VARIANT 1
 /* ADSG_TUNE_RHS_KRONECKER = 1 (default 0; 3D; the autotuner leaves it): forms without a k
@@ -342,7 +343,7 @@ int adsg_time_phases(adsg_sim* h, int nsteps, const adsg_rhs_form* form, const i
  * owns and storing the others in a spill array (allocated with the handle, about one to
  * three values per element), which a second kernel adds in a fixed order. Both are
  * deterministic; the sums are grouped differently (equal to rounding). The autotuner times
- * both. The 2D element loop is one launch of strips that share no DOF with either value (and
+ * both in 3D. The 2D element loop is one launch of strips that share no DOF with either value (and
  * in batches, whose problems therefore equal the same problems run alone); there the tiling is
  * that of the k-field gradients. Default 1 in 3D and for 2D meshes of at most 2048 tiles of
  * 16 x 16 elements, 0 for larger 2D meshes. */
