@@ -204,11 +204,10 @@ template <typename T>
 constexpr bool rhs3_march_kfield(int p) {
     return sizeof(T) == sizeof(double) || p < 3;
 }
-// its 32-bit byte offsets within a plane of DOFs
-constexpr bool rhs3_march_fits(int bytes, long nx, long ny) {
-    return nx * ny * bytes < (1L << 32);
-}
 void rhs3_march_tiles(int p, int bytes, bool kfield, const int elements[3], int tile[3], int nt[3]);
+// whether its launch can take the mesh: 32-bit byte offsets within a plane of DOFs, and a grid of
+// fewer than 2^32 lanes
+bool rhs3_march_fits(int p, int bytes, bool kfield, const int elements[3]);
 template <typename T>
 hipError_t launch_rhs3_march(int p, const T* u_prev, T* rhs, const dev_tables<T>* dirs, const rhs_params<T>& prm,
                              const int tile[3], const int nt[3], hipStream_t s);

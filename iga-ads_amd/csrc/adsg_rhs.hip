@@ -1613,8 +1613,8 @@ hipError_t rhs_fields(int dim, const T* up, T* rhs, const dev_tables<T>* d,
     if (dim == 3 && variant == 5 && !rhs3_col_supported<T>(P, prm)) variant = P == 3 ? 2 : 1;
     // element columns on the matrix cores where the form allows, else the degree's default
     // per-element variant
-    const bool march = dim == 3 && rhs3_march_fits(sizeof(T), d[0].dofs, d[1].dofs) &&
-                       (!kf || rhs3_march_kfield<T>(P));
+    const int el[3] = {d[0].elements, d[1].elements, d[2].elements};
+    const bool march = dim == 3 && (!kf || rhs3_march_kfield<T>(P)) && rhs3_march_fits(P, sizeof(T), kf, el);
     const bool one = dim == 3 && (code & kRhsOneLaunch) != 0 && prm.spill && variant != 3 && variant != 5 &&
                      (!kf || march);
     // 3D in one launch: the marching kernel for variant 4 and for every form with a k field,
