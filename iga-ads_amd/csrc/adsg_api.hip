@@ -992,26 +992,27 @@ int adsg::create_sim(const adsg_config* cfg, hipStream_t shared, bool vectors, a
         h->dirs[d].slots.push_back(std::move(s0));
     }
     // default element-kernel variant (adsg_autotune refines it): the one measured fastest for
-    // the degree, precision and size. In one launch variant 4 is the marching kernel: a tile of
+    // the degree, precision and mesh. In one launch variant 4 is the marching kernel: a tile of
     // it marches through its elements plane by plane, so it needs elements enough to fill the
-    // device with short marches; below, the per-element kernels finish sooner. Crossovers (step
-    // times, cubes and 77 x 101 x 61): p = 3 between 40^3 (FP64 variant 2 27 against 31 us per
-    // element pass, FP32 variant 1 20 against 23) and 48^3 (60 against 50, 37 against 29); p = 2
-    // FP64 between 64^3 (31 against 34) and 77 x 101 x 61 (60 against 57), FP32 between 96^3 (55
-    // against 58) and 128^3 (113 against 88); p = 1 between 96^3 (31 against 31; FP32 22 against
-    // 24) and 128^3 (59 against 53; 38.2 against 37.7). 3D handles start with the one-launch
-    // tiling (ADSG_TUNE_RHS_TILING), which was faster for every variant measured; so do 2D
-    // handles of at most 2048 tiles of 16 x 16 elements, whose colour launches are too small to
-    // fill the device (128^2 p = 2 with a k field: 0.046 -> 0.029 ms per step). Larger 2D
-    // meshes keep the colour launches, as the batches do (with thousands of tiles per launch
-    // the fix-up pass costs more than the colour tails it removes).
+    // device with short marches; below, and on meshes its tiles fit badly, the per-element kernels
+    // finish sooner (rhs3_march_pays): at p = 3 variant 2 (FP32 variant 1 up to 512 tiles of 8 x 8 x
+    // 3 elements, two per compute unit: 32^3 37 against 41 us a step; 17 x 70 x 60, 540 tiles, 70
+    // against 57, 5 x 300 x 300 179 against 150, 36 x 50 x 60 57 against 60), else variant 1. 3D handles start with the one-launch
+    // tiling (ADSG_TUNE_RHS_TILING), which was faster for every variant measured. In 2D the tiling
+    // is that of the k-field gradients: one launch for handles of at most 2048 tiles of 16 x 16
+    // elements, whose colour launches are too small to fill the device; larger ones keep the
+    // colour launches (with thousands of tiles per launch the fix-up pass costs more than the
+    // colour tails it removes).
     {
-        long E = 1;
-        for (int d = 0; d < h->dim; ++d) E *= h->dirs[d].tab.elements;
         const int p = dc[0]->p;
         const bool f32 = h->precision == ADSG_FP32;
-        const long march = p == 3 ? 1L << 16 : f32 ? 1L << 20 : p == 2 ? 3L << 17 : 1L << 20;
-        h->rhs_variant = E >= march ? 4 : p == 3 && !f32 ? 2 : 1;
+        long tiles = 1;
+        for (int d = 0; d < h->dim; ++d) tiles *= (h->dirs[d].tab.elements + (d == 2 ? 2 : 7)) / (d == 2 ? 3 : 8);
+        h->rhs_variant = p == 3 && (!f32 || tiles > 512) ? 2 : 1;
+        if (h->dim == 3 && !h->general) {
+            const int el[3] = {h->dirs[0].tab.elements, h->dirs[1].tab.elements, h->dirs[2].tab.elements};
+            if (adsg::rhs3_march_pays(p, f32 ? 4 : 8, false, el)) h->rhs_variant = 4;
+        }
         h->rhs_col_shape = 1;  // variant 5: two columns per wave, one chunk per workgroup
         const long tiles16 = static_cast<long>((h->dirs[0].tab.elements + 15) / 16) * ((h->dirs[1].tab.elements + 15) / 16);
         h->rhs_tiling = h->general ? 0 : h->dim == 3 || tiles16 <= 2048 ? 1 : 0;

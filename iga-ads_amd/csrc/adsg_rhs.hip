@@ -1616,10 +1616,10 @@ hipError_t rhs_fields(int dim, const T* up, T* rhs, const dev_tables<T>* d,
     const int el[3] = {d[0].elements, d[1].elements, d[2].elements};
     const bool march = dim == 3 && (!kf || rhs3_march_kfield<T>(P)) && rhs3_march_fits(P, sizeof(T), kf, el);
     const bool one = dim == 3 && (code & kRhsOneLaunch) != 0 && prm.spill && variant != 3 && variant != 5 &&
-                     (!kf || march);
-    // 3D in one launch: the marching kernel for variant 4 and for every form with a k field,
-    // which the per-element kernels take in colour launches only (70 x 50 x 61, p = 2, FP64: 34 us
-    // against 154 us in eight launches and a fill)
+                     (!kf || (march && rhs3_march_pays(P, sizeof(T), true, el)));
+    // 3D in one launch: the marching kernel for variant 4 and, where it is faster, for forms with a
+    // k field, which the per-element kernels take in colour launches only (70 x 50 x 61, p = 2,
+    // FP64: 34 us against 154 us in eight launches and a fill)
     const bool marched = dim == 2 || (march && one && (kf || variant == 4));
     if (one && variant == 4 && !marched) variant = P == 3 ? 2 : 1;
     const long n = static_cast<long>(d[0].dofs) * d[1].dofs * (dim == 3 ? d[2].dofs : 1);
@@ -1773,6 +1773,45 @@ long rhs_spill_slots(int dim, int p, const int elements[3]) {
         default:
             return 0;
     }
+}
+
+// Modelled times, us: the march takes its cost in planes times kPlane; the per-element kernels in
+// one launch a time per tile (kStart: the difference of what neither grows with), the colour launches
+// at least kLaunch each, more with many tiles. A march pads x to 31 / 19 / 16 elements and y to 4, the
+// tiles x and y to 8, so on thin meshes and those just over a tile the element count alone chose
+// wrongly. Fitted to the step times of 39 meshes per degree and
+// precision (32^3 to 160^3, 1 to 39 or 130 to 300 elements along x, 1 to 17 along y or z; p = 3 FP64 68):
+// the kernel chosen is 0.02 to 0.65 % slower than the faster one on average, 8 % at most (by
+// element count 5 % in FP64 for p = 2 and 3, 82 % at most; with a k field always marching 3 %, 53 %
+// at most). Examples, march against per-element: 128^3 FP64 p = 1 96 / 101, p = 2 176 / 229, p = 3
+// 389 / 759; 8 x 256 x 256 p = 2 FP64 119 / 92; 17 x 140 x 140 p = 2 FP64 68 / 82; 5 x 300 x 300
+// p = 3 FP64 335 / 256, with a k field 433 against 314 in colours. One element along x or y takes the
+// colour launches of p = 3 half as long again as two.
+bool rhs3_march_pays(int p, int bytes, bool kfield, const int elements[3]) {
+    if (p < 1 || p > 3) return false;
+    const int f32 = bytes == 4;
+    int tile[3], nt[3];
+    const double cost = rhs3_march_tiles(p, bytes, kfield, elements, tile, nt);
+    const int te[3] = {8, 8, p == 3 ? 3 : 4};  // tile<3, p>
+    double tiles = 1, launches = 1;
+    for (int d = 0; d < 3; ++d) {
+        const int n = (elements[d] + te[d] - 1) / te[d];
+        tiles *= n;
+        if (n > 1) launches *= 2;
+    }
+    if (!kfield) {
+        static const double kPlane[2][4] = {{0, 1.0, 2.2, 3.8}, {0, 0.71, 1.5, 2.4}};
+        static const double kTile[2][4] = {{0, 5.4e-3, 20e-3, 57e-3}, {0, 3.3e-3, 11e-3, 32e-3}};
+        static const double kStart[2][4] = {{0, -1.7, -8.2, -25}, {0, -0.36, -5.2, -13}};
+        return kPlane[f32][p] * cost + kStart[f32][p] < kTile[f32][p] * tiles;
+    }
+    if (p == 3 && (elements[0] == 1 || elements[1] == 1)) return true;
+    static const double kPlane[2][4] = {{0, 1.1, 1.2, 3.6}, {0, 1.0, 1.7, 3.6}};
+    static const double kLaunch[2][4] = {{0, 4.6, 17, 30}, {0, 4.5, 9.5, 30}};
+    static const double kOverlap[2][4] = {{0, 2.3, 8.5, 20}, {0, 2.25, 4.75, 20}};
+    static const double kTile[2][4] = {{0, 6e-3, 21e-3, 64e-3}, {0, 6e-3, 12.5e-3, 64e-3}};
+    return kPlane[f32][p] * cost <
+           launches * std::max(kLaunch[f32][p], kOverlap[f32][p] + kTile[f32][p] * tiles / launches);
 }
 
 void rhs2_batch_tiles(int elements_x, int elements_y, int ntx2[4], int count[4]) {

@@ -459,7 +459,7 @@ __global__ __launch_bounds__((64 * kMarchRows), march_waves(sizeof(T), P, KF)) v
 }
 
 template <int P>
-void march_tiles(int waves, const int el[3], int tile[3]) {
+double march_tiles(int waves, const int el[3], int tile[3]) {  // its cost, in planes (rhs3_march_pays)
     tile[0] = march<P>::TX;
     tile[1] = kMarchRows;
     // elements per workgroup along z. A workgroup's cost is its elements plus about 2P for the
@@ -477,16 +477,18 @@ void march_tiles(int waves, const int el[3], int tile[3]) {
             tile[2] = tz;
         }
     }
+    return best;
 }
 
 }  // namespace
 
-void rhs3_march_tiles(int p, int bytes, bool kfield, const int elements[3], int tile[3], int nt[3]) {
+double rhs3_march_tiles(int p, int bytes, bool kfield, const int elements[3], int tile[3], int nt[3]) {
     const int waves = march_waves(bytes, p, kfield);
-    if (p == 1) march_tiles<1>(waves, elements, tile);
-    if (p == 2) march_tiles<2>(waves, elements, tile);
-    if (p == 3) march_tiles<3>(waves, elements, tile);
+    const double cost = p == 1   ? march_tiles<1>(waves, elements, tile)
+                        : p == 2 ? march_tiles<2>(waves, elements, tile)
+                                 : march_tiles<3>(waves, elements, tile);
     for (int d = 0; d < 3; ++d) nt[d] = (elements[d] + tile[d] - 1) / tile[d];
+    return cost;
 }
 
 bool rhs3_march_fits(int p, int bytes, bool kfield, const int elements[3]) {

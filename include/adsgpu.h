@@ -314,8 +314,9 @@ int adsg_time_phases(adsg_sim* h, int nsteps, const adsg_rhs_form* form, const i
  * wave (p <= 2; 2 at p = 3));
  * they compute the same sums (variants 2 and 4 add them in other orders; in FP64 variant 3
  * equals 1, or 2 at p = 3, bit for bit). A new handle starts with the variant measured
- * fastest for its degree, precision and element count (4 from 2^16 elements at p = 3, 3 * 2^17
- * at p = 2 in FP64 and 2^20 otherwise; below, 2 for FP64 p = 3 and else 1).
+ * fastest for its degree, precision and mesh (4 on large meshes that its tiles fit, cubes from
+ * about 60, 50 and 33 elements a side on for p = 1, 2 and 3 in FP64, 90, 90 and 41 in FP32; else 2
+ * for p = 3, in FP32 beyond 512 tiles of 8 x 8 x 3 elements, and 1).
  * ADSG_TUNE_SWEEP_VARIANT selects the line sweep (0: lines cut into segments solved by
  * separate waves and joined through FP64-computed influence coefficients, where the factors
  * are unpivoted and the lines are 1..16 segments of at most 32 rows long (up to 512 DOFs),
@@ -339,8 +340,9 @@ int adsg_time_phases(adsg_sim* h, int nsteps, const adsg_rhs_form* form, const i
  * wave, bit 1 three chunks of 16 DOF planes per workgroup; the autotuner times all four. */
 #define ADSG_TUNE_RHS_COLUMNS 4
 /* ADSG_TUNE_RHS_TILING (3D variants 0, 1, 2 and 4; forms with a k field run variant 4's
- * kernel then, in FP32 for p <= 2): 0 = 8 parity-colour launches, whose tiles share no DOF; 1 = one launch over all tiles, each tile adding the entries of its DOF block that it
- * owns and storing the others in a spill array (allocated with the handle, about one to
+ * kernel then, in FP32 for p <= 2, unless the mesh is so thin that the colour launches are
+ * faster): 0 = 8 parity-colour launches, whose tiles share no DOF; 1 = one launch over all tiles,
+ * each tile adding the entries of its DOF block that it owns and storing the others in a spill array (allocated with the handle, about one to
  * three values per element), which a second kernel adds in a fixed order. Both are
  * deterministic; the sums are grouped differently (equal to rounding). The autotuner times
  * both in 3D. The 2D element loop is one launch of strips that share no DOF with either value (and
