@@ -34,6 +34,37 @@ def f_elem(d, p):
     return 2 * c * 2 * n ** (d + 1) + (d + 2) * n ** d
 
 
+def f_march3(p, f32, mass):
+    """Flops per element of k_rhs3_march: per x Gauss point (a lane) and DOF plane its stages U, Y,
+    Z, T, S (adsg_rhs_march.hip), the sums of S over the elements and waves left out; idle lanes
+    and the planes and rows that neighbouring tiles repeat are not counted."""
+    m = p + 1
+    if f32:  # differences instead of the first term of each sum, FP64 sums across elements
+        u = 5 * p * m + 3 * p
+        y = m * 2 * (2 * p + m)
+        z = m * (1 + 3 * p) + m * m * 2 * ((2 if mass else 1) * p + 2 * m + (4 if mass else 3) * m) + 3 * m * m
+    else:
+        u = 2 * 2 * m * m
+        y = 2 * 3 * m * m
+        z = m * m * 2 * (4 + 4 if mass else 3 + 3) * m
+    z += (2 if mass else 0) * m * m  # the integrand
+    return m * (u + y + z + 2 * 3 * m * m + 2 * 2 * m * m)
+
+
+def f_march2(p, f32):
+    """Flops per element of k_rhs2_march with a reaction term, counted like f_march3."""
+    m = p + 1
+    x = p + 4 * p * m + m * (1 + 3 * p)
+    y = m * m * (2 * (2 * p + m) + 5 + 6 * m)
+    s = 2 * m * m + 4 * m ** 3 + m * m if f32 else 4 * m * m + 2 * m
+    return x + y + s + m
+
+
+def f_rhs3(p, variant, tiling, f32, mass):
+    """Flops per element of the 3D element kernel that a handle with these settings runs."""
+    return f_march3(p, f32, mass) if variant == 4 and tiling == 1 else f_elem(3, p)
+
+
 def run_form(ag, precision, ne, steps, warmup, u0, dt, variant=None, kron=False):
     """Plain explicit heat step (c2 form) in the given precision: autotune, warm up, time
     `steps` graph-replayed steps, then time the phases of 3 eager steps. kron: the rhs of
@@ -137,7 +168,8 @@ def implicit_block(ag, np, ne, steps, warmup):
                      f"A = (x)_d (M_d + dt/2 K_d); natural BC"),
         "fp64": {"value": N * steps / t64, "ms_per_step": 1e3 * t64 / steps, "phases_ms": ph64,
                  "rhs_variant": v64,
-                 "rhs_tflops": f_elem(3, 3) * ne ** 3 / (ph64["rhs"] * 1e-3) / 1e12},
+                 "rhs_tflops": f_rhs3(3, v64, sim64.get_tuning(ag.TUNE_RHS_TILING), False, False) * ne ** 3
+                 / (ph64["rhs"] * 1e-3) / 1e12},
     }
     for name, flags in (("fp32", 0), ("fp32_refined", ag.STEP_REFINE)):
         s32, t32, ph32, x32, v32 = run_implicit(ag, ag.FP32, ne, steps, warmup, u0, f, dt, flags)
@@ -215,7 +247,6 @@ def ensemble_block(ag, np, count, steps, dt):
     u0 = [wl.smooth_unit(q["p"], q["ne"], q["seed"]) for q in probs]
     dofs = sum(u.size for u in u0)
     elems = sum(q["ne"] ** 2 for q in probs)
-    flops = sum(f_elem(2, q["p"]) * q["ne"] ** 2 for q in probs)
     out, res = {}, {}
     for name, prec in (("fp32", ag.FP32), ("fp64", ag.FP64)):
         tc0 = time.perf_counter()
@@ -239,6 +270,8 @@ def ensemble_block(ag, np, count, steps, dt):
         t = time.perf_counter() - t0
         out[name] = [b.get(i) for i in range(len(probs))]
         b.close()
+        flops = sum((f_march2(q["p"], prec == ag.FP32) if tile == 0 else f_elem(2, q["p"])) * q["ne"] ** 2
+                    for q in probs)
         res[name] = {"value": dofs * steps / t, "ms_per_step": 1e3 * t / steps,
                      "setup_ms": {"create": 1e3 * (tc1 - tc0), "prepare": 1e3 * (tc2 - tc1),
                                   "in_steps": (tc2 - tc0) / (t / steps),
@@ -527,7 +560,8 @@ def main():
     rhs_kernel = {3: "k_rhs3_pipe", 4: "k_rhs3_march" if til64 == 1 else "k_rhs3_zpair"}.get(var64, "k_rhs3")
     one = til64 == 1 and var64 != 3
     launches = 1 if one else 8
-    launch_flops = f_elem(3, 2) * E / launches
+    flops_per_element = f_rhs3(2, var64, til64, False, True)
+    launch_flops = flops_per_element * E / launches
     launch_ms = ph64["rhs"] / launches
     traffic_key = rhs_kernel + (" (one launch)" if one else "")
     launch_desc = ("one launch over all tiles; its spill fix-up k_rhs_fixup (memory-bound, "
@@ -566,9 +600,10 @@ def main():
             "launch_flops": launch_flops,
             "launch_ms": launch_ms,
             "note": ("FP64 vector-ALU bound (MI355X FP64 vector peak = FP64 matrix peak = "
-                     "78.6 TFLOP/s); achieved = 3051 flop/element x the elements of one launch "
-                     "(E, or E/8 per colour launch) / average launch time (HIP events around the "
-                     "phase's launches on the handle's stream); traffic = HBM bytes per launch "
+                     f"78.6 TFLOP/s); achieved = {flops_per_element} flop/element (the operations of "
+                     "the kernel that runs, without idle lanes and what neighbouring tiles repeat) x "
+                     "the elements of one launch (E, or E/8 per colour launch) / average launch time "
+                     "(HIP events around the phase's launches on the handle's stream); traffic = HBM bytes per launch "
                      "from rocprofv3 FETCH_SIZE and WRITE_SIZE scaled by a copy-kernel "
                      "calibration"),
         },
@@ -593,7 +628,8 @@ def main():
         ti, phi, xi, vari = run_increment_form(ag, ag.FP64, ne, args.steps, args.warmup, u0, dt)
         err = float(np.linalg.norm(x32 - x64) / np.linalg.norm(x64))
         kern32 = {3: "k_rhs3_pipe", 4: "k_rhs3_march" if til32 == 1 else "k_rhs3_zpair"}.get(var32, "k_rhs3")
-        tf32 = f_elem(3, 2) * E / (ph32["rhs"] * 1e-3) / 1e12
+        flops32 = f_rhs3(2, var32, til32, True, False)
+        tf32 = flops32 * E / (ph32["rhs"] * 1e-3) / 1e12
         result["forms"] = {
             "fp64": {"value": value, "ms_per_step": ms_step},
             "fp64_increment": {
@@ -620,11 +656,12 @@ def main():
                     "kernel": f"{kern32} (FP32, variant {var32}, tiling {til32})",
                     "bound": "valu_fp32",
                     "achieved": tf32, "unit": "TFLOP/s",
-                    "peak": 78.6, "frac": tf32 / 78.6,
+                    "peak": rates["valu_fp32"], "frac": tf32 / rates["valu_fp32"],
                     "peak_mfma_fp32": 157.3, "frac_of_mfma_fp32": tf32 / 157.3,
-                    "note": ("3051 flop/element x E elements / the rhs phase's time; "
-                             "FP32 VALU without packed instructions issues at the FP64 rate "
-                             "(78.6 TFLOP/s); 157.3 TFLOP/s is the FP32 MFMA / packed peak"),
+                    "note": (f"{flops32} flop/element (counted like the FP64 kernel's, its FP64 sums "
+                             "across elements included) x E elements / the rhs phase's time; peak = "
+                             "plain FP32 FMAs as measured on this device (device_rates_tflops), "
+                             "157.3 TFLOP/s is the FP32 MFMA / packed peak"),
                 },
             },
         }
