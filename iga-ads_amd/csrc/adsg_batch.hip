@@ -776,8 +776,8 @@ int adsg_batch_autotune(adsg_batch* b, double* ms_out) {
     (void)hipEventCreate(&e0);
     (void)hipEventCreate(&e1);
     // every (element kernel, line grouping) pair: strips or 8 x 8 element tiles; lines either
-    // segmented (64 lines per workgroup of nine waves) or one lane per line (64 lines per
-    // one-wave workgroup)
+    // segmented (workgroups of nine waves, which take as many groups of 64 lines as their segments
+    // fit) or one lane per line (64 lines per one-wave workgroup)
     int best = b->shape, best_sweep = b->sweep, rc = ADSG_OK;
     float best_ms = 1e30f;
     for (int shape = 0; shape <= 1 && rc == ADSG_OK; ++shape) {

@@ -297,8 +297,8 @@ int adsg_check_finite(adsg_sim* h, int which);
  * (examples/scalability/test3d.hpp:67-101). Averages per step in milliseconds: ms[0] the
  * element-loop kernels (the colour launches, or the one launch over all tiles),
  * ms[1] boundary handling, ms[2], ms[3], ms[4] line sweeps in x, y, z, ms[5] the whole step,
- * ms[6] the start of the rhs (a source's load vector scaled in; the zero fill, where one is
- * needed, is part of ms[0]). With the one-launch tiling the spill fix-up, and the FP64
+ * ms[6] the start of the separable rhs (ADSG_TUNE_RHS_KRONECKER: a source's load vector scaled in;
+ * in the element loop that, and the zero fill where one is needed, are part of ms[0]). With the one-launch tiling the spill fix-up, and the FP64
  * boundary zeroing with it, run at the start of the x sweep and count in ms[2]; without
  * the fix-up the FP64 zeroing is done by the x sweep as it loads its lines. */
 int adsg_time_phases(adsg_sim* h, int nsteps, const adsg_rhs_form* form, const int* slots, int flags,
@@ -395,8 +395,9 @@ int adsg_batch_step(adsg_batch* b, int nsteps);
 int adsg_batch_synchronize(adsg_batch* b);
 /* ADSG_TUNE_BATCH_TILE: element kernel of the batch, 0 = strips of every problem in one
  * launch, 1 = tiles of 8 x 8 elements, one launch per degree and parity colour.
- * ADSG_TUNE_SWEEP_VARIANT: 0 = segmented line sweeps (9 waves per 64 lines; used when every
- * problem's lines split into segments), 1 = one lane per line.
+ * ADSG_TUNE_SWEEP_VARIANT: 0 = segmented line sweeps (workgroups of 9 waves, which take as many
+ * groups of 64 lines as their segments fit; used when every problem's lines split into segments),
+ * 1 = one lane per line.
  * adsg_batch_autotune times one step with each element kernel and each line grouping (the two
  * sweep variants), keeps the fastest pair and restores the state; ms_out[0..1] (may be
  * NULL) receives each element kernel's time with its better sweep variant. */
