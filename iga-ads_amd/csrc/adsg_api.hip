@@ -1011,7 +1011,9 @@ int adsg::create_sim(const adsg_config* cfg, hipStream_t shared, bool vectors, a
         h->rhs_variant = p == 3 && (!f32 || tiles > 512) ? 2 : 1;
         if (h->dim == 3 && !h->general) {
             const int el[3] = {h->dirs[0].tab.elements, h->dirs[1].tab.elements, h->dirs[2].tab.elements};
-            if (adsg::rhs3_march_pays(p, f32 ? 4 : 8, false, el)) h->rhs_variant = 4;
+            int tile[3], nt[3];
+            const double cost = adsg::rhs3_march_tiles(p, f32 ? 4 : 8, false, el, tile, nt);
+            if (adsg::rhs3_march_pays(p, f32 ? 4 : 8, false, el, cost)) h->rhs_variant = 4;
         }
         h->rhs_col_shape = 1;  // variant 5: two columns per wave, one chunk per workgroup
         const long tiles16 = static_cast<long>((h->dirs[0].tab.elements + 15) / 16) * ((h->dirs[1].tab.elements + 15) / 16);

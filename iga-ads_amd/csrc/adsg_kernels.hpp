@@ -206,12 +206,14 @@ constexpr bool rhs3_march_kfield(int p) {
 }
 // (returns their modelled cost, in planes marched by rounds of the workgroups that run at once)
 double rhs3_march_tiles(int p, int bytes, bool kfield, const int elements[3], int tile[3], int nt[3]);
-// whether its launch can take the mesh: 32-bit byte offsets within a plane of DOFs, and a grid of
-// fewer than 2^32 lanes
-bool rhs3_march_fits(int p, int bytes, bool kfield, const int elements[3]);
-// whether it is the faster kernel for the mesh: against the per-element kernels in one launch, or,
-// with a k field, in colour launches
-bool rhs3_march_pays(int p, int bytes, bool kfield, const int elements[3]);
+// whether its launch can take the mesh (nt tiles): 32-bit byte offsets within a plane of DOFs, and a
+// grid of fewer than 2^32 lanes, 256 per tile
+constexpr bool rhs3_march_fits(int bytes, long nx, long ny, const int nt[3]) {
+    return nx * ny * bytes < (1L << 32) && static_cast<long>(nt[0]) * nt[1] * nt[2] < (1L << 24);
+}
+// whether it is the faster kernel for the mesh, cost being its tiles': against the per-element kernels
+// in one launch, or, with a k field, in colour launches
+bool rhs3_march_pays(int p, int bytes, bool kfield, const int elements[3], double cost);
 template <typename T>
 hipError_t launch_rhs3_march(int p, const T* u_prev, T* rhs, const dev_tables<T>* dirs, const rhs_params<T>& prm,
                              const int tile[3], const int nt[3], hipStream_t s);

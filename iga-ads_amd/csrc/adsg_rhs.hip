@@ -1447,12 +1447,10 @@ hipError_t rhs3_one(const T* up, T* rhs, const dev_tables<T>* d, const rhs_param
 // Variant 4 in one launch: the marching kernel (adsg_rhs_march.hip) on its own tiles, then
 // the spill fix-up over the DOFs.
 template <typename T, int P>
-hipError_t rhs3_march(const T* up, T* rhs, const dev_tables<T>* d, const rhs_params<T>& prm, hipStream_t s) {
-    const int el[3] = {d[0].elements, d[1].elements, d[2].elements};
-    int tl[3], nt[3];
-    if (el[0] <= 0 || el[1] <= 0 || el[2] <= 0) return hipSuccess;
+hipError_t rhs3_march(const T* up, T* rhs, const dev_tables<T>* d, const rhs_params<T>& prm, const int tl[3],
+                      const int nt[3], hipStream_t s) {
+    if (d[0].elements <= 0 || d[1].elements <= 0 || d[2].elements <= 0) return hipSuccess;
     if (!prm.spill) return hipErrorInvalidValue;
-    rhs3_march_tiles(P, sizeof(T), prm.kfield != nullptr, el, tl, nt);
     rhs_params<T> q = prm;
     const int n[3] = {d[0].dofs, d[1].dofs, d[2].dofs};
     for (int i = 0; i < 3; ++i)
@@ -1613,14 +1611,20 @@ hipError_t rhs_fields(int dim, const T* up, T* rhs, const dev_tables<T>* d,
     if (dim == 3 && variant == 5 && !rhs3_col_supported<T>(P, prm)) variant = P == 3 ? 2 : 1;
     // element columns on the matrix cores where the form allows, else the degree's default
     // per-element variant
-    const int el[3] = {d[0].elements, d[1].elements, d[2].elements};
-    const bool march = dim == 3 && (!kf || rhs3_march_kfield<T>(P)) && rhs3_march_fits(P, sizeof(T), kf, el);
-    const bool one = dim == 3 && (code & kRhsOneLaunch) != 0 && prm.spill && variant != 3 && variant != 5 &&
-                     (!kf || (march && rhs3_march_pays(P, sizeof(T), true, el)));
+    bool one = dim == 3 && (code & kRhsOneLaunch) != 0 && prm.spill && variant != 3 && variant != 5;
     // 3D in one launch: the marching kernel for variant 4 and, where it is faster, for forms with a
     // k field, which the per-element kernels take in colour launches only (70 x 50 x 61, p = 2,
     // FP64: 34 us against 154 us in eight launches and a fill)
-    const bool marched = dim == 2 || (march && one && (kf || variant == 4));
+    bool march = one && (kf ? rhs3_march_kfield<T>(P) : variant == 4);
+    int tl[3], nt[3];
+    if (march) {
+        const int el[3] = {d[0].elements, d[1].elements, d[2].elements};
+        const double cost = rhs3_march_tiles(P, sizeof(T), kf, el, tl, nt);
+        march = rhs3_march_fits(sizeof(T), d[0].dofs, d[1].dofs, nt) &&
+                (!kf || rhs3_march_pays(P, sizeof(T), true, el, cost));
+    }
+    one = one && (!kf || march);
+    const bool marched = dim == 2 || march;
     if (one && variant == 4 && !marched) variant = P == 3 ? 2 : 1;
     const long n = static_cast<long>(d[0].dofs) * d[1].dofs * (dim == 3 ? d[2].dofs : 1);
     bool overwrite = (code & kRhsOverwrite) != 0;
@@ -1638,7 +1642,7 @@ hipError_t rhs_fields(int dim, const T* up, T* rhs, const dev_tables<T>* d,
         if (e != hipSuccess) return e;
     }
     if (dim == 3) {
-        if (marched) return rhs3_march<T, P>(up, rhs, d, prm, s);
+        if (marched) return rhs3_march<T, P>(up, rhs, d, prm, tl, nt, s);
         if (variant == 5) return launch_rhs3_col<T>(P, up, rhs, d, prm, (code >> 4) & 15, s);
         if (variant == 1) return rhs3_fields<T, P, 1>(up, rhs, d, prm, one, s);
         if (variant == 2) return rhs3_fields<T, P, 2>(up, rhs, d, prm, one, s);
@@ -1787,11 +1791,9 @@ long rhs_spill_slots(int dim, int p, const int elements[3]) {
 // 389 / 759; 8 x 256 x 256 p = 2 FP64 119 / 92; 17 x 140 x 140 p = 2 FP64 68 / 82; 5 x 300 x 300
 // p = 3 FP64 335 / 256, with a k field 433 against 314 in colours. One element along x or y takes the
 // colour launches of p = 3 half as long again as two.
-bool rhs3_march_pays(int p, int bytes, bool kfield, const int elements[3]) {
+bool rhs3_march_pays(int p, int bytes, bool kfield, const int elements[3], double cost) {
     if (p < 1 || p > 3) return false;
     const int f32 = bytes == 4;
-    int tile[3], nt[3];
-    const double cost = rhs3_march_tiles(p, bytes, kfield, elements, tile, nt);
     const int te[3] = {8, 8, p == 3 ? 3 : 4};  // tile<3, p>
     double tiles = 1, launches = 1;
     for (int d = 0; d < 3; ++d) {

@@ -491,21 +491,14 @@ double rhs3_march_tiles(int p, int bytes, bool kfield, const int elements[3], in
     return cost;
 }
 
-bool rhs3_march_fits(int p, int bytes, bool kfield, const int elements[3]) {
-    int tile[3], nt[3];
-    rhs3_march_tiles(p, bytes, kfield, elements, tile, nt);
-    return (static_cast<long>(elements[0]) + p) * (elements[1] + p) * bytes < (1L << 32) &&
-           static_cast<long>(nt[0]) * nt[1] * nt[2] * (64 * kMarchRows) < (1L << 32);
-}
-
 namespace {
 
 template <typename T, int P, bool KF, int FM>
 hipError_t march_launch(const T* up, T* rhs, const dev_tables<T>* d, const rhs_params<T>& prm, const int tile[3],
                         const int nt[3], hipStream_t s) {
     const long blocks = static_cast<long>(nt[0]) * nt[1] * nt[2];
-    const int el[3] = {d[0].elements, d[1].elements, d[2].elements};
-    if (tile[0] != march<P>::TX || tile[1] != kMarchRows || tile[2] < P || !rhs3_march_fits(P, sizeof(T), KF, el))
+    if (tile[0] != march<P>::TX || tile[1] != kMarchRows || tile[2] < P ||
+        !rhs3_march_fits(sizeof(T), d[0].dofs, d[1].dofs, nt))
         return hipErrorInvalidValue;
     march_args<T> a;
     a.up = up;
