@@ -463,7 +463,8 @@ double march_tiles(int waves, const int el[3], int tile[3]) {  // its cost, in p
     tile[0] = march<P>::TX;
     tile[1] = kMarchRows;
     // elements per workgroup along z. A workgroup's cost is its elements plus about 2P for the
-    // planes without an element at its ends and its start; `cap` workgroups run at once, and the
+    // planes without an element at its ends and its start; `cap` workgroups run at once (the waves
+    // that march_waves asks for; p = 1 and FP32 up to p = 2 fit 4 to 8 per compute unit), and the
     // last ones to start leave half a round partly idle. Fewer than 4 elements lost everywhere.
     const long columns = static_cast<long>((el[0] + tile[0] - 1) / tile[0]) * ((el[1] + tile[1] - 1) / tile[1]);
     const double cap = 256.0 * waves;
